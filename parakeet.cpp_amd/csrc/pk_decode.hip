@@ -411,8 +411,7 @@ struct pk_decoder {
     float chain_ep_ms = 0.f, chain_loop_ms = 0.f;
     int chain_iters = 0;
     int lock_fd = -1;          // this GPU's cross-process loop lock (see DeviceLoopLock), -1: none
-    const void *loop_fn[2] = {};   // the decode-loop instantiations for this decoder's weight storage:
-                                   // several domains, one domain (argmax key slots)
+    const void *loop_fn = nullptr;   // the decode-loop instantiation for this decoder's weight storage
     // Drop every device and pinned allocation without freeing it (process exit).
     void forget_device() {
         for (DevBuf *b : {&arena, &eproj, &slots_h, &slots_c, &slots_pp, &slots_r, &slots_ctrl, &special, &d_desc,
@@ -747,36 +746,25 @@ PK_API int pk_decoder_create(const pk_decoder_desc *d, int32_t n_slots, pk_decod
         // PK_GEMV=1 (comparisons only): all-q8_0 decoders run the instantiation with the
         // wavefront-reduction GEMV form for column tiles of at most 4 live utterances
         const char *gv = std::getenv("PK_GEMV");
-        if (all_q8 && gv && gv[0] == '1') {
-            dec->loop_fn[0] = reinterpret_cast<const void *>(decode_loop_kernel<pkdev::kWcQ8Gemv, false>);
-            dec->loop_fn[1] = reinterpret_cast<const void *>(decode_loop_kernel<pkdev::kWcQ8Gemv, true>);
-        } else {
-            dec->loop_fn[0] = all_q8 ? reinterpret_cast<const void *>(decode_loop_kernel<kWcQ8, false>)
-                            : all_half ? reinterpret_cast<const void *>(decode_loop_kernel<kWcHalf, false>)
-                                       : reinterpret_cast<const void *>(decode_loop_kernel<kWcAny, false>);
-            dec->loop_fn[1] = all_q8 ? reinterpret_cast<const void *>(decode_loop_kernel<kWcQ8, true>)
-                            : all_half ? reinterpret_cast<const void *>(decode_loop_kernel<kWcHalf, true>)
-                                       : reinterpret_cast<const void *>(decode_loop_kernel<kWcAny, true>);
-        }
+        dec->loop_fn = all_q8 && gv && gv[0] == '1' ? reinterpret_cast<const void *>(decode_loop_kernel<kWcQ8Gemv>)
+                       : all_q8                     ? reinterpret_cast<const void *>(decode_loop_kernel<kWcQ8>)
+                       : all_half                   ? reinterpret_cast<const void *>(decode_loop_kernel<kWcHalf>)
+                                                    : reinterpret_cast<const void *>(decode_loop_kernel<kWcAny>);
     }
-    size_t stat = 0;   // the larger static LDS of the two instantiations
-    for (const void *fn : dec->loop_fn) {
-        hipFuncAttributes fa{};
-        if (hipFuncGetAttributes(&fa, fn) != hipSuccess) return cleanup(fail(PK_ERR_DEVICE, "hipFuncGetAttributes"));
-        stat = std::max(stat, fa.sharedSizeBytes);
-    }
+    const void *fn = dec->loop_fn;
+    hipFuncAttributes fa{};
+    if (hipFuncGetAttributes(&fa, fn) != hipSuccess) return cleanup(fail(PK_ERR_DEVICE, "hipFuncGetAttributes"));
+    const size_t stat = fa.sharedSizeBytes;
     const size_t need = (size_t)dec->lds_block > stat ? (size_t)dec->lds_block - stat : 0;
     if (dec->lds_fixed + (size_t)2 * kWaves * kWave * 16 > need)
         return cleanup(fail(PK_ERR_UNSUPPORTED, "LDS %zu B needed, %d available", dec->lds_fixed + stat,
                             dec->lds_block));
     dec->lds_bytes = need;
-    for (const void *fn : dec->loop_fn) {
-        if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need) != hipSuccess)
-            return cleanup(fail(PK_ERR_DEVICE, "hipFuncSetAttribute"));
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, need) != hipSuccess || per_cu < 1)
-            return cleanup(fail(PK_ERR_DEVICE, "decode kernel does not fit on a CU"));
-    }
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need) != hipSuccess)
+        return cleanup(fail(PK_ERR_DEVICE, "hipFuncSetAttribute"));
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, need) != hipSuccess || per_cu < 1)
+        return cleanup(fail(PK_ERR_DEVICE, "decode kernel does not fit on a CU"));
     dec->nwg = std::min(dec->n_cu, kBlock);
     if ((rc = scratch_address(dec->device, &dec->scratch))) return cleanup(rc);
     dec->lock_fd = open_loop_lock(dec->device);
@@ -1083,7 +1071,7 @@ int launch_loop(pk_decoder *dec, int nwg, KParams &p, size_t lds, bool coop) {
     }
     prev = dec->stream;
     void *args[] = {&p};
-    const void *fn = dec->loop_fn[p.slots ? 1 : 0];   // one domain: the argmax-slot instantiation
+    const void *fn = dec->loop_fn;
     bool &refused = g_loops.coop_refused[dec->device];
     // 0: cooperative, 1: ordinary dispatch, -1: the default above.  Under a profiler (its
     // ROCPROF* environment, or its tool library preloaded) always an ordinary dispatch.
@@ -1277,20 +1265,22 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
     const int *d_dom_wg = reinterpret_cast<const int *>(put(pl.dom_wg.data(), 4 * pl.dom_wg.size()));
     HIP_TRY(hipMemcpyAsync(d_desc, hd, desc_bytes, hipMemcpyHostToDevice, dec->stream));
 
-    // argmax shards: about 8 ranks per shard
-    p.shards = 1;
-    while (p.shards < pkdev::kShards && p.shards * 8 < pl.P) p.shards *= 2;
-    const size_t keys_bytes = (size_t)2 * pl.n_dom * pkdev::kColCap * p.shards * 2 * 8;
-    // one-domain launches: per-workgroup argmax key slots (used while at most
-    // kSlotCols joint columns are live); PK_ARGMAX_SLOTS=0 keeps the sharded
-    // atomics and barrier instead (for comparisons)
-    const char *slots_env = std::getenv("PK_ARGMAX_SLOTS");
-    const bool use_slots = pl.n_dom == 1 && !(slots_env && slots_env[0] == '0');
-    const size_t slots_bytes = use_slots ? (size_t)2 * pl.P * pkdev::kSlotCols * 2 * 8 : 0;
+    // column capacity of the argmax keys, row capacities of the exchange buffers (powers of two;
+    // h rows at least 8, a whole 128-byte line per unit tile)
+    const int dom_max = *std::max_element(pl.dom_n.begin(), pl.dom_n.end());
+    p.cols = dom_max > kTile ? 2 * kTile : kTile;
+    p.prows = 1;
+    while (p.prows < dom_max) p.prows *= 2;
+    p.rows = std::max(p.prows, 8);
+    const size_t keys_bytes = (size_t)2 * pl.n_dom * (pl.P + 2) * p.cols * 8;
+    // the ranks that own duration rows V1 .. Vo-1 (at most two neighbouring tiles)
+    p.n_durk = 0;
+    if (p.Dn > 0)
+        for (int t = p.V1 / kTile; t <= (p.Vo - 1) / kTile; ++t) p.dur_rank[p.n_durk++] = t % pl.P;
     // the words every launch starts from zero, in one allocation cleared by
-    // one fill: 64 B of status, the barrier flags, the argmax keys and slots
+    // one fill: 64 B of status, the barrier flags, the argmax keys
     const size_t flags_bytes = (size_t)nwg * kFlagStride * 4,
-                 clear_bytes = 256 + flags_bytes + keys_bytes + slots_bytes;
+                 clear_bytes = 256 + flags_bytes + keys_bytes;
     void *d_clear = nullptr;
     if ((rc = cs.get(dec->d_clear, clear_bytes, &d_clear))) return rc;
     // (one fill kernel, never a memset, so that the call may run under graph capture)
@@ -1387,22 +1377,23 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
     p.wg_rank = d_wg_rank;
     p.dom_wg = d_dom_wg;
     void *d_xchg = nullptr;
-    const size_t xh = 2 * (size_t)L * m * H, xp = (size_t)m * J, xr = 2 * (size_t)L * m * 4 * H;
+    // a one-domain launch of at most kSmallB utterances never exchanges h_0
+    p.hl0 = pl.n_dom == 1 && m <= kSmallB ? 1 : 0;
+    const size_t xs = (size_t)L * m * H, xc = 2 * (size_t)m * H, xr = 2 * (size_t)m * 4 * H,
+                 xh = 2 * (size_t)(L - p.hl0) * pl.n_dom * H * p.rows, xp = 2 * (size_t)pl.n_dom * J * p.prows;
+    const size_t xchg = (xs + xc + xr + xh + xp) * 4;
     // the loop addresses the exchange buffers with 32-bit buffer offsets
-    if ((2 * xh + xp + xr) * 4 >= (1ull << 31))
-        return fail(PK_ERR_UNSUPPORTED, "exchange buffers of %d utterances exceed 2 GiB", m);
-    if ((rc = cs.get(dec->d_xchg, (2 * xh + xp + xr) * 4, &d_xchg))) return rc;
-    p.hx = static_cast<float *>(d_xchg);
-    p.cx = p.hx + xh;
-    p.ppx = p.cx + xh;
-    p.rx = p.ppx + xp;
-    p.xchg_bytes = (unsigned)((2 * xh + xp + xr) * 4);
+    if (xchg >= (1ull << 31)) return fail(PK_ERR_UNSUPPORTED, "exchange buffers of %d utterances exceed 2 GiB", m);
+    if ((rc = cs.get(dec->d_xchg, xchg, &d_xchg))) return rc;
+    p.hs = static_cast<float *>(d_xchg);
+    p.cx = p.hs + xs;
+    p.rx = p.cx + xc;
+    p.hx = p.rx + xr;
+    p.ppx = p.hx + xh;
+    p.xchg_bytes = (unsigned)xchg;
     p.status = static_cast<int *>(d_clear) + 4;
     p.flags = reinterpret_cast<unsigned *>(static_cast<uint8_t *>(d_clear) + 256);
     p.keys = reinterpret_cast<unsigned long long *>(static_cast<uint8_t *>(d_clear) + 256 + flags_bytes);
-    p.slots = slots_bytes ? reinterpret_cast<unsigned long long *>(static_cast<uint8_t *>(d_clear) + 256 +
-                                                                 flags_bytes + keys_bytes)
-                          : nullptr;
     // PK_PROFILE_PHASES=1: workgroup 0 accumulates per-phase wall-clock time (stderr summary)
     const bool prof = !cs.fixed && getenv("PK_PROFILE_PHASES") != nullptr;
     p.prof = nullptr;
@@ -1591,8 +1582,8 @@ relaunch:
     if (prof) {
         unsigned long long t[pkdev::kPrN];
         HIP_TRY(hipMemcpy(t, dec->d_prof.p, sizeof t, hipMemcpyDeviceToHost));
-        static const char *names[pkdev::kPrN] = {"L0", "sync0", "L1", "sync1", "pred", "sync2",
-                                                 "J-stage", "J-compute", "J-sync", "decide", "stageLSTM"};
+        static const char *names[pkdev::kPrN] = {"L0", "stage-h0", "L1", "stage-h1", "pred", "J-stage", "J-compute",
+                                                 "keys", "decide"};
         double total = 0;
         for (double v : t) total += v;
         fprintf(stderr, "[pk phases] %d iterations, %d domains x %d wg, total %.3f ms:", status[1], pl.n_dom, pl.P,

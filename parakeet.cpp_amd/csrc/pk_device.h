@@ -24,13 +24,11 @@ constexpr int kSmallB = 4;                  // LSTM batch at or below which laye
 constexpr int kIdxBits = 14;                // argmax key: index field
 constexpr int kStampShift = 46;             // argmax key: 14 index + 32 value bits below the stamp
 constexpr unsigned kMaxStamp = (1u << 18) - 1;
-constexpr int kFlagStride = 64;             // words between barrier flags (256 B)
+constexpr int kFlagStride = 32;             // words between barrier flags (128 B, one L2 line)
 // error word of a launch whose ordinary dispatch was not co-resident (never returned to a caller:
 // the host relaunches the call cooperatively)
 constexpr int kStatusNotResident = 0x7001;
-constexpr int kShards = 32;                 // argmax keys: most max targets per utterance and head
-constexpr int kSlotCols = 2;                // one-domain launches with at most this many joint columns
-                                            // exchange argmax keys through per-workgroup slots
+constexpr unsigned kEmpty = 0xffffffffu;     // exchange word not written yet (a NaN no producer stores)
 constexpr int kKPad = 8;                    // halves of padding per staged row (bank spread)
 
 // Flags in the per-utterance control word.
@@ -114,12 +112,19 @@ struct KParams {
                                  // iteration, copied to the row of the step that takes the column
     const int *reset;            // nullable [n_utts]: 1 = fresh state whatever the slot holds
     int *ctrl_out;               // nullable [n_utts][PK_CTRL_N]: control words after the call
-    // exchange buffers of one launch (batch-indexed, written/read coherently)
-    float *hx;           // [2][L][n][H] ping-pong by utterance parity
-    float *cx;           // [2][L][n][H]
-    float *ppx;          // [n][J]
-    float *rx;           // [2][L][n][4H]  W_hh . h (no bias), unit-major rows, ping-pong like hx
-    unsigned xchg_bytes; // hx, cx, ppx, rx: one allocation in this order, from hx
+    // exchange buffers of one launch (one allocation from hs, xchg_bytes long; coherent accesses).
+    // State by batch index, read and written by the workgroup that owns the units except where
+    // layer 0 runs redundantly:
+    float *hs;           // [L][n][H]      h of every layer (for the slots at the end)
+    float *cx;           // [2][n][H]      c of layer 0, ping-pong by utterance parity
+    float *rx;           // [2][n][4H]     W_hh0 . h0 (no bias), unit-major rows, ping-pong like cx
+    // Data every workgroup of a domain waits for, word by word (kEmpty until written):
+    float *hx;           // [L - hl0][2][n_dom][H/4][rows][4]  h of one LSTM step by list position; the
+                         // 4 units x rows of a tile are one producer's whole lines
+    float *ppx;          // [2][n_dom][J/16][prows][16]  b_p + W_p . h by domain utterance and parity
+    int rows, prows;     // row capacities (powers of two >= utterances per domain; rows >= 8)
+    int hl0;             // first layer of hx: 1 where layer 0 always runs redundantly
+    unsigned xchg_bytes;
     // domains: independent utterance groups, each on dom_size workgroups
     int n_dom, dom_size, nt;
     const int *dom_n;            // [n_dom] utterances per domain
@@ -129,8 +134,11 @@ struct KParams {
     const int *dom_wg;           // [n_dom][dom_size] workgroup of each rank
     // sync
     unsigned *flags;             // [nwg * kFlagStride]
-    unsigned long long *keys;    // [2][n_dom][kColCap][shards][2] best keys per joint column, by iteration parity
-    int shards;                  // power of two <= kShards: ranks per shard ~ 8
+    // argmax keys by iteration parity, stamped with the iteration: each workgroup's best token key
+    // per joint column, and the duration keys of the one or two ranks that own duration rows
+    unsigned long long *keys;    // [2][n_dom][P][cols] then [2][n_dom][2][cols]
+    int cols;                    // column capacity: 16 or 32
+    int dur_rank[2], n_durk;     // ranks that own duration rows (n_durk of them)
     int *status;                 // [0] error code, [1] iterations, [2] overflow, [3] trace overflow,
                                  // [9] co-residency decision (cleared per launch)
     unsigned arrive_ticks;       // ordinary dispatch: limit of the arrival wait (100 MHz ticks); 0: none
@@ -141,14 +149,11 @@ struct KParams {
     int bias_floats;             // LDS bias table size (floats)
     int wcache_bytes;            // LDS weight cache per workgroup (0: weights are read from L2)
     unsigned long long *prof;    // nullable: per-phase wall-clock totals of workgroup 0 (100 MHz ticks)
-    unsigned long long *slots;   // nullable (one-domain launches): [2][P][kSlotCols][2] stamped best keys
-                                 // of each workgroup, by iteration parity
 };
 
 // Phase timers (workgroup 0 only, when p.prof is set): totals kept in LDS,
 // written to p.prof when the loop ends.
-enum { kPrL0 = 0, kPrSync0, kPrL1, kPrSync1, kPrPred, kPrSync2, kPrJStage, kPrJCompute, kPrJSync, kPrDecide,
-       kPrStageL, kPrN };
+enum { kPrL0 = 0, kPrStage0, kPrL1, kPrStage1, kPrPred, kPrJStage, kPrJCompute, kPrKeys, kPrDecide, kPrN };
 
 // ---------------------------------------------------------------- memory helpers
 
@@ -552,8 +557,10 @@ __global__ void __launch_bounds__(256) enc_proj_narrow_kernel(const _Float16 *__
 struct Ctl {                      // per-workgroup copy of its domain's control state
     int b[kDomCap];               // batch index of each domain utterance
     int t[kDomCap], T[kDomCap], sym[kDomCap], pend[kDomCap], flags[kDomCap];
-    int ntok[kDomCap], steps[kDomCap], nseg[kDomCap], segst[kDomCap], last[kDomCap], cur[kDomCap];
+    int ntok[kDomCap], steps[kDomCap], nseg[kDomCap], segst[kDomCap], last[kDomCap];
+    int cur[kDomCap];             // parity of the utterance's state once its pending token (if any) is taken
     int lst[kDomCap], jst[kDomCap];
+    int stp[kDomCap];             // 1: the utterance took an LSTM step in this launch
     // joint columns: column i < nj is joint-list utterance i at its frame t; columns
     // sbase[i] .. sbase[i] + sn[i] - 1 are the same utterance at frames t + 1 .. t + sn[i]
     int cu[kColCap], co[kColCap], sbase[kDomCap], sn[kDomCap];
@@ -566,12 +573,14 @@ struct Ctl {                      // per-workgroup copy of its domain's control 
     int tbase[kDomCap];           // tokens before this call (EOU segment indices)
     int dur[PK_MAX_DURATIONS];    // duration values (the decision step reads them from LDS)
     int n, nl, nj;
+    int lgn;                      // log2 of the LSTM list length, rounded up
     int dom, rank, P;
+    int ok;                       // 0: a wait ended without its data (error or time-out)
     // this workgroup's tiles of an LSTM matrix, of W_p and of W_o (fixed for the
     // launch; computed once, since each is an integer division)
     int own_lstm, own_pred, own_out;
     int pass[PK_MAX_LAYERS + 1];  // items per pass of the phase consuming layer l's output (l < L), of W_o (L)
-    unsigned mag_p, mag_h, mag_units;   // udiv multipliers for P, H and 4 * own_lstm
+    unsigned mag_p;               // udiv multiplier for P
     unsigned wmask;               // bit ul: this workgroup writes utterance ul's outputs (ul % P == rank)
     int tq_n, tq_col[kColCap], tq_b[kColCap], tq_step[kColCap];   // logit tap: (column, utterance, step)
                                                                   // of this iteration's decisions
@@ -670,7 +679,9 @@ __device__ __forceinline__ void build_lists(Ctl &s, bool spec) {
             total = __shfl(incl, kWave - 1, kWave);
         }
         if (lane == 0) {
-            s.nl = __popcll(bl);
+            const int nl = __popcll(bl);
+            s.nl = nl;
+            s.lgn = nl <= 1 ? 0 : 32 - __builtin_clz((unsigned)(nl - 1));
             s.nj = nj;
             s.ncol = nj + total;
         }
@@ -678,104 +689,137 @@ __device__ __forceinline__ void build_lists(Ctl &s, bool spec) {
     lds_sync();
 }
 
-// Domain barrier: every member publishes its epoch in its own flag word and
-// every member polls all members' flags (thread t polls rank t).  No
-// cache-wide fences: cross-workgroup data is stored and loaded coherently
-// (SC1), and each thread waits for its own stores (s_waitcnt 0) before
-// arriving.  Returns false if the error word is set or the wait exceeds ~2 s.
-__device__ __forceinline__ bool dom_sync(const KParams &p, const Ctl &s, unsigned &epoch) {
+// A wait that does not end by itself: every 64 polls the error word and the
+// clock are read, and after ~2 s the launch ends with PK_ERR_TIMEOUT (s.ok is
+// checked once per iteration; waits that follow end at their 64th poll).
+__device__ __forceinline__ bool wait_over(const KParams &p, Ctl &s, unsigned &n, unsigned long long &t0) {
+    if ((++n & 63u) != 0u) return false;
+    const unsigned long long now = __builtin_amdgcn_s_memrealtime();   // 100 MHz
+    if (t0 == 0ull) t0 = now;
+    if (__hip_atomic_load(p.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+        s.ok = 0;
+        return true;
+    }
+    if (now - t0 > 200000000ull) {
+        __hip_atomic_store(p.status, PK_ERR_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s.ok = 0;
+        return true;
+    }
+    return false;
+}
+
+// Domain barrier before the first iteration: every member publishes its epoch
+// in its own flag word and every member polls all members' flags (thread t
+// polls rank t).  No cache-wide fences: cross-workgroup data is stored and
+// loaded coherently (SC1), and each thread waits for its own stores
+// (s_waitcnt 0) before arriving.  Returns false if the error word is set or the
+// wait exceeds ~2 s.
+__device__ __forceinline__ bool dom_sync(const KParams &p, Ctl &s, unsigned &epoch) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    __shared__ int s_ok;
     ++epoch;
-    if (threadIdx.x == 0) {
-        s_ok = 1;
+    if (threadIdx.x == 0)
         __hip_atomic_store(p.flags + (size_t)blockIdx.x * kFlagStride, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
     if (threadIdx.x < s.P) {
-        // tight poll; the error word and the clock are checked every 64 polls
         unsigned *f = p.flags + (size_t)p.dom_wg[s.dom * s.P + threadIdx.x] * kFlagStride;
-        const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
         unsigned n = 0;
-        while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
-            if ((++n & 63) != 0) continue;
-            if (__hip_atomic_load(p.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) { s_ok = 0; break; }
-            if (__builtin_amdgcn_s_memrealtime() - t0 > 200000000ull) {   // 100 MHz clock: 2 s
-                __hip_atomic_store(p.status, PK_ERR_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s_ok = 0;
-                break;
-            }
-        }
+        unsigned long long t0 = 0ull;
+        while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch)
+            if (wait_over(p, s, n, t0)) break;
     }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __syncthreads();
-    return s_ok != 0;
+    return s.ok != 0;
 }
 
-// Exchange-buffer offsets (floats).
-__device__ __forceinline__ size_t hx_off(const KParams &p, int buf, int layer, int b) {
-    return (((size_t)buf * p.L + layer) * p.n_utts + b) * p.H;
+// Exchange between the workgroups of a domain inside an iteration.
+//
+// Every value that other workgroups need (h of each layer, the prediction
+// output, the argmax keys) is waited for word by word: a consumer loads the
+// words it stages until none of them is empty.  One device-coherent store and
+// the load that sees it replace the store, its acknowledgement, a barrier (flag
+// store, polls of every member's flag) and the staging load behind it.  Layouts
+// give each producer whole lines: a tile's rows are stored by one wave, so no
+// line is invalidated under its readers by another workgroup's store.
+// Measured per exchange with nothing else in flight (store, wait, staged rows):
+// 16 rows over 64 workgroups 1.84 us against 2.71 us with a barrier, over 16
+// workgroups 2.07 against 2.57, one row over 256 workgroups 1.75 against 2.15.
+//
+// Words become empty again in time: h of an LSTM step sits in one of two halves
+// (hx), and its producer empties the half of the previous step when the next one
+// begins; the prediction output of an utterance sits in the half of its parity
+// (ppx), and its producer empties the old half when it writes the new one.  By
+// then every reader is done: the argmax keys are exchanged at the end of each
+// iteration, and a workgroup stores its keys after its last staging.  It also
+// waits for all of its own stores before that, so a workgroup that has seen
+// every key sees every word emptied or written in the iteration.
+
+// State offsets (floats): c_0 / h_0 of parity buf, W_hh0 . h_0.
+__device__ __forceinline__ size_t cx_off(const KParams &p, int buf, int b) { return ((size_t)buf * p.n_utts + b) * p.H; }
+__device__ __forceinline__ size_t rx_off(const KParams &p, int buf, int b) {
+    return ((size_t)buf * p.n_utts + b) * 4 * p.H;
 }
-__device__ __forceinline__ size_t rx_off(const KParams &p, int buf, int layer, int b) {
-    return (((size_t)buf * p.L + layer) * p.n_utts + b) * 4 * p.H;
+__device__ __forceinline__ size_t hs_off(const KParams &p, int layer, int b) {
+    return ((size_t)layer * p.n_utts + b) * p.H;
+}
+// Exchange offsets (floats): the 4 units of tile t for list row u; the 16 rows
+// of pred tile t for domain utterance ul.
+__device__ __forceinline__ unsigned hx_at(const KParams &p, int dom, int layer, int half, int t, int u) {
+    return ((((unsigned)((layer - p.hl0) * 2 + half) * p.n_dom + dom) * (p.H / 4) + t) * p.rows + u) * 4u;
+}
+__device__ __forceinline__ unsigned ppx_at(const KParams &p, int dom, int half, int t, int ul) {
+    return ((((unsigned)half * p.n_dom + dom) * (p.J / kTile) + t) * p.prows + ul) * (unsigned)kTile;
+}
+// A produced word: never the empty pattern (a NaN that loses one payload bit).
+__device__ __forceinline__ float filled(float v) {
+    const unsigned b = __float_as_uint(v);
+    return __uint_as_float(b == kEmpty ? b - 1u : b);
+}
+__device__ __forceinline__ bool has_empty(float4 v) {
+    return max(max(__float_as_uint(v.x), __float_as_uint(v.y)),
+               max(__float_as_uint(v.z), __float_as_uint(v.w))) == kEmpty;
+}
+__device__ __forceinline__ float4 empty4() {
+    const float e = __uint_as_float(kEmpty);
+    return make_float4(e, e, e, e);
 }
 
-struct Bufs {
-    __amdgpu_buffer_rsrc_t hx, cx, ppx, rx, ep, encp;
-};
-
-// One utterance's slot state in float4 chunks: h of every layer, c_0, pp,
-// R_0 (c and R of layers >= 1 live in the LDS state during a launch).  Chunk
-// q is at `slot` in its slot array and at float offset `x` from p.hx in the
-// exchange buffers (hx, cx, ppx, rx are consecutive).
-struct StateChunk {
-    float *slot;
-    long long x;
-};
-__device__ __forceinline__ int state_chunks(const KParams &p) { return (p.L * p.H + p.H + p.J + 4 * p.H) / 4; }
-__device__ __forceinline__ StateChunk state_chunk(const KParams &p, int q, int slot, int b, int buf) {
-    const int H = p.H, L = p.L, J = p.J;
-    int i = 4 * q;
-    if (i < L * H) {
-        const int l = i / H;
-        return {p.slot_h + (size_t)slot * L * H + i, (long long)hx_off(p, buf, l, b) + (i - l * H)};
-    }
-    i -= L * H;
-    if (i < H) return {p.slot_c + (size_t)slot * L * H + i, (long long)(p.cx - p.hx) + (long long)hx_off(p, buf, 0, b) + i};
-    i -= H;
-    if (i < J) return {p.slot_pp + (size_t)slot * J + i, (long long)(p.ppx - p.hx) + (long long)b * J + i};
-    i -= J;
-    return {p.slot_r + (size_t)slot * L * 4 * H + i, (long long)(p.rx - p.hx) + (long long)rx_off(p, buf, 0, b) + i};
-}
 constexpr int kCopyB = 4;   // float4 per thread in flight when copying state
 
-// Stage vectors of length K for n <= 16 utterances into an activation block:
-// row u <- src(off(u)) via coherent loads; rows n .. 15 are zero.  Every
-// thread issues all of its loads before converting any of them.
-// Staging: 32 threads per row, so a 512-thread block covers 16 rows per
-// round; each thread resolves its row once and moves float4 chunks sub,
-// sub + 32, ... (kStageMax per thread in flight: 160 float4 = K 640 per pass).
-constexpr int kStageMax = 5, kStageTpr = 32;
-template <class OffFn>
-__device__ __forceinline__ void stage_act(const Act &x, int K, int n, __amdgpu_buffer_rsrc_t r, OffFn off) {
-    const int per = K / 4, sub = threadIdx.x % kStageTpr;
-    for (int u0 = 0; u0 < n; u0 += kBlock / kStageTpr) {
-        const int u = u0 + threadIdx.x / kStageTpr;
-        const bool live = u < n;
-        const unsigned row = (unsigned)(off(live ? u : n - 1) * 4);   // byte offset of the row
-        for (int k0 = 0; k0 < per; k0 += kStageTpr * kStageMax) {
+struct Bufs {
+    __amdgpu_buffer_rsrc_t hx, cx, ppx, rx, ep, encp, keys;
+};
+
+// Staging: loads of kStageMax float4 per thread in flight; a thread converts
+// and drops each as it arrives and loads the rest again.
+constexpr int kStageMax = 5;
+
+// h of layer lc for list rows c0 .. c0+nc-1 (nc <= 16) into an activation block.
+// A wave covers 4 tiles x 16 rows (16 tiles x 4 rows for short lists): 1 KB in a
+// row of the exchange buffer.
+__device__ __forceinline__ void stage_h(const KParams &p, Ctl &s, const Bufs &B, const Act &x, int lc, int half,
+                                        int c0, int nc) {
+    const int lg = nc <= 4 ? 2 : 4;
+    const int u = threadIdx.x & ((1 << lg) - 1), t0 = threadIdx.x >> lg, step = kBlock >> lg, ntile = p.H / 4;
+    const unsigned base = hx_at(p, s.dom, lc, half, 0, c0 + u) * 4u, stride = (unsigned)p.rows * 16u;
+    for (int b0 = 0; b0 < ntile; b0 += step * kStageMax) {
+        unsigned pend = 0u, n = 0u;
+        unsigned long long since = 0ull;
+#pragma unroll
+        for (int j = 0; j < kStageMax; ++j)
+            if (u < nc && b0 + t0 + step * j < ntile) pend |= 1u << j;
+        while (pend != 0u) {
             float4 v[kStageMax];
 #pragma unroll
-            for (int j = 0; j < kStageMax; ++j) {
-                const int k4 = k0 + sub + kStageTpr * j;
-                v[j] = ld4_coh(r, live && k4 < per ? row + (unsigned)k4 * 16 : kBad);
-            }
+            for (int j = 0; j < kStageMax; ++j)
+                v[j] = ld4_coh(B.hx, (pend >> j) & 1u ? base + (unsigned)(b0 + t0 + step * j) * stride : kBad);
 #pragma unroll
-            for (int j = 0; j < kStageMax; ++j) {
-                const int k4 = k0 + sub + kStageTpr * j;
-                if (live && k4 < per) put4(x, u, k4 * 4, v[j]);
-            }
+            for (int j = 0; j < kStageMax; ++j)
+                if (((pend >> j) & 1u) && !has_empty(v[j])) {
+                    put4(x, u, (b0 + t0 + step * j) * 4, v[j]);
+                    pend &= ~(1u << j);
+                }
+            if (pend != 0u && wait_over(p, s, n, since)) break;
         }
     }
 }
@@ -1245,37 +1289,27 @@ __device__ __forceinline__ void cache_matrix(const TMat &m, int rank, int P, uns
     }
 }
 
-// A one-domain launch with at most kSlotCols joint columns exchanges the argmax
-// keys through per-workgroup slots instead of atomics, a barrier and a gather:
-// each workgroup stores its stamped best key per column and head in its own
-// slot, and every workgroup polls all slots until each carries this
-// iteration's stamp (the stamp is the arrival signal).  One round trip instead
-// of two.  The condition is the same in every workgroup of the domain; ONE
-// launches (one domain, p.slots set) run their own instantiation of the loop.
-template <bool ONE>
-__device__ __forceinline__ bool slot_mode(const Ctl &s) {
-    return ONE && s.ncol <= kSlotCols;
-}
-
 // Joint + argmax for this workgroup's output tiles.  Utterances are processed
 // 16 at a time (one MFMA column tile).
-// The encp rows of the joint's first staging round (column tile 0, chunks
-// sub, sub + 32, ...), loaded at the start of the iteration: the list rebuild
-// has fixed every column's frame, and the loads complete during layer 0, whose
-// own loads take as long, instead of at the joint's staging.
+// Row mapping of the joint's staging: a wave covers one pred tile (16 values)
+// of 16 columns, 1 KB in a row of ppx; thread t takes column (t / 4) % 16,
+// values 4 (t % 4) .. +3 of pred tiles t / 64, t / 64 + 8, ...
+// The encp rows of the first round (column tile 0) are loaded at the start of
+// the iteration: the list rebuild has fixed every column's frame, and the loads
+// complete during layer 0, whose own loads take as long, instead of at the
+// joint's staging.
 __device__ __forceinline__ void encp_prefetch(const KParams &p, const Ctl &s, const Bufs &B, float4 (&e)[kStageMax]) {
-    const int J = p.J, per = J / 4, sub = threadIdx.x % kStageTpr, u = threadIdx.x / kStageTpr;
-    const int nc = min(kTile, s.ncol);
-    const bool live = u < nc;
+    const int J = p.J, ntile = J / kTile, g = threadIdx.x & 3, u = (threadIdx.x >> 2) & 15, t0 = threadIdx.x >> 6;
+    const bool live = u < min(kTile, s.ncol);
     const unsigned erow = (unsigned)((size_t)s.crow[live ? u : 0] * J * 4);
 #pragma unroll
     for (int j = 0; j < kStageMax; ++j) {
-        const int k4 = sub + kStageTpr * j;
-        e[j] = ld4(B.encp, live && k4 < per ? erow + (unsigned)k4 * 16 : kBad);
+        const int t = t0 + kWaves * j;
+        e[j] = ld4(B.encp, live && t < ntile ? erow + (unsigned)(t * kTile + g * 4) * 4 : kBad);
     }
 }
 
-template <int WC, bool ONE>
+template <int WC>
 __device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs &B, const Lds &S, unsigned stamp,
                             const float4 (&epre)[kStageMax], unsigned long long &tlast) {
     const int J = p.J, lane = threadIdx.x & (kWave - 1);
@@ -1285,36 +1319,43 @@ __device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs
         const int nc = min(kTile, s.ncol - c0);
         Act x = S.act[0];
         x.n = nc;
-        // stage hidden = relu(encp[t] + pp) for this column tile (row mapping as in stage_act)
+        // stage hidden = relu(encp[t] + pp) for this column tile
         {
-            const int per = J / 4, sub = threadIdx.x % kStageTpr;
-            for (int u0 = 0; u0 < nc; u0 += kBlock / kStageTpr) {
-                const int u = u0 + threadIdx.x / kStageTpr;
-                const bool live = u < nc;
-                const int col = c0 + (live ? u : nc - 1);
-                const unsigned erow = (unsigned)((size_t)s.crow[col] * J * 4);
-                const unsigned prow = (unsigned)((size_t)s.cb[col] * J * 4);
-                for (int k0 = 0; k0 < per; k0 += kStageTpr * kStageMax) {
-                    float4 e[kStageMax], q[kStageMax];
+            const int ntile = J / kTile, g = threadIdx.x & 3, u = (threadIdx.x >> 2) & 15, t0 = threadIdx.x >> 6;
+            const bool live = u < nc;
+            const int col = c0 + (live ? u : 0), ul = s.cu[col];
+            const unsigned erow = (unsigned)((size_t)s.crow[col] * J * 4);
+            const unsigned prow = (ppx_at(p, s.dom, s.cur[ul], 0, ul) + g * 4) * 4u;
+            const unsigned stride = (unsigned)p.prows * kTile * 4u;
+            for (int b0 = 0; b0 < ntile; b0 += kWaves * kStageMax) {
+                float4 e[kStageMax];
+                unsigned pend = 0u, n = 0u;
+                unsigned long long since = 0ull;
 #pragma unroll
-                    for (int j = 0; j < kStageMax; ++j) {
-                        const int k4 = k0 + sub + kStageTpr * j;
-                        const bool ok = live && k4 < per;
-                        e[j] = (c0 == 0 && k0 == 0) ? epre[j] : ld4(B.encp, ok ? erow + (unsigned)k4 * 16 : kBad);
-                        q[j] = ld4_coh(B.ppx, ok ? prow + (unsigned)k4 * 16 : kBad);
-                    }
+                for (int j = 0; j < kStageMax; ++j) {
+                    const int t = b0 + t0 + kWaves * j;
+                    const bool ok = live && t < ntile;
+                    e[j] = (c0 == 0 && b0 == 0) ? epre[j]
+                                                : ld4(B.encp, ok ? erow + (unsigned)(t * kTile + g * 4) * 4 : kBad);
+                    if (ok) pend |= 1u << j;
+                }
+                while (pend != 0u) {
+                    float4 q[kStageMax];
 #pragma unroll
-                    for (int j = 0; j < kStageMax; ++j) {
-                        const int k4 = k0 + sub + kStageTpr * j;
-                        if (live && k4 < per) {
+                    for (int j = 0; j < kStageMax; ++j)
+                        q[j] = ld4_coh(B.ppx, (pend >> j) & 1u ? prow + (unsigned)(b0 + t0 + kWaves * j) * stride : kBad);
+#pragma unroll
+                    for (int j = 0; j < kStageMax; ++j)
+                        if (((pend >> j) & 1u) && !has_empty(q[j])) {
                             float4 v = make_float4(e[j].x + q[j].x, e[j].y + q[j].y, e[j].z + q[j].z, e[j].w + q[j].w);
                             v.x = (0.0f < v.x) ? v.x : 0.0f;
                             v.y = (0.0f < v.y) ? v.y : 0.0f;
                             v.z = (0.0f < v.z) ? v.z : 0.0f;
                             v.w = (0.0f < v.w) ? v.w : 0.0f;
-                            put4(x, u, k4 * 4, v);
+                            put4(x, u, (b0 + t0 + kWaves * j) * kTile + g * 4, v);
+                            pend &= ~(1u << j);
                         }
-                    }
+                    if (pend != 0u && wait_over(p, s, n, since)) break;
                 }
             }
         }
@@ -1371,31 +1412,28 @@ __device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs
             if (best0) atomicMax(&s.wgkey[c0 + u][0], best0);
             if (best1) atomicMax(&s.wgkey[c0 + u][1], best1);
         }
+        // the keys stored next say that this workgroup's other stores of the iteration have landed
+        if (c0 + kTile >= s.ncol) __builtin_amdgcn_s_waitcnt(0);
         lds_sync();
         TLA(27);
         pmark(p, s, tlast, kPrJCompute);
     }
-    if (slot_mode<ONE>(s)) {   // this workgroup's stamped best keys into its own slot
-        if (threadIdx.x < 2 * s.ncol) {
-            const int u = threadIdx.x / 2, head = threadIdx.x % 2;
-            __hip_atomic_store(p.slots + (((size_t)(stamp & 1) * s.P + s.rank) * kSlotCols + u) * 2 + head,
-                               ((unsigned long long)stamp << kStampShift) | s.wgkey[u][head], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        }
-        TLA(28);
-        return;
-    }
-    // one device-scope max per utterance and head into shard rank % kShards
-    // (spreads the atomics of many workgroups over several words); the stamp
-    // keeps keys of iteration `stamp` above every older key in the same parity
-    unsigned long long *keys = p.keys + (size_t)(stamp & 1) * p.n_dom * kColCap * p.shards * 2;
+    // this workgroup's stamped best token key of every joint column, one line per
+    // workgroup; the duration keys from the ranks that own duration rows
     if (threadIdx.x < 2 * s.ncol) {
-        const int u = threadIdx.x / 2, head = threadIdx.x % 2;
-        const unsigned long long k = s.wgkey[u][head];
-        if (k != 0ull)
-            __hip_atomic_fetch_max(&keys[((size_t)(s.dom * kColCap + u) * p.shards + (s.rank & (p.shards - 1))) * 2 + head],
-                                   ((unsigned long long)stamp << kStampShift) | k, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+        const int u = threadIdx.x >> 1, head = threadIdx.x & 1;
+        const unsigned long long k = ((unsigned long long)stamp << kStampShift) | s.wgkey[u][head];
+        const size_t par = stamp & 1;
+        if (head == 0) {
+            __hip_atomic_store(p.keys + ((par * p.n_dom + s.dom) * s.P + s.rank) * p.cols + u, k, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            for (int d = 0; d < p.n_durk; ++d)
+                if (p.dur_rank[d] == s.rank)
+                    __hip_atomic_store(p.keys + (size_t)2 * p.n_dom * s.P * p.cols +
+                                           ((par * p.n_dom + s.dom) * 2 + d) * p.cols + u,
+                                       k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
     TLA(28);
 }
@@ -1403,51 +1441,49 @@ __device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs
 // Layer 0 from the precomputed input projection: gates = E'[token] + R0,
 // elementwise per unit.  redundant: every unit for every listed utterance,
 // h' also written into the layer-1 activation block; otherwise only this
-// workgroup's unit tiles.
+// workgroup's unit tiles.  Work item: unit g of list row u of a tile, so a wave
+// stores whole tiles of the exchange buffer.
 // Owners store h', c' coherently.
 // Each thread issues the loads of up to kL0 units before computing any.
 constexpr int kL0 = 3;
-__device__ __forceinline__ void lstm_layer0(const KParams &p, Ctl &s, const Lds &S, const Bufs &B, bool redundant) {
-    const int H = p.H;
-    const int n_own = s.own_lstm;
-    const int nunits = redundant ? H : 4 * n_own;
-    const unsigned mag = redundant ? s.mag_h : s.mag_units;
-    const int n_work = s.nl * nunits;
+__device__ __forceinline__ void lstm_layer0(const KParams &p, Ctl &s, const Lds &S, const Bufs &B, bool redundant,
+                                            int half) {
+    const int H = p.H, lgn = s.lgn, nl = s.nl;
+    const int n_work = (redundant ? H / 4 : s.own_lstm) << (lgn + 2);
     for (int base = 0; base < n_work; base += kL0 * kBlock) {
         float4 e[kL0], r[kL0];
         float c_prev[kL0];
-        int uq[kL0], jq[kL0];
 #pragma unroll
         for (int q = 0; q < kL0; ++q) {   // no branches: unused loads take kBad and return 0
             const int i = base + threadIdx.x + q * kBlock;
-            const int ic = min(i, n_work - 1);
-            const int u = udiv(ic, mag, nunits), jj = ic - u * nunits;   // ic * nunits < 2^32 (H <= 4096)
-            const int j = redundant ? jj : 4 * (s.rank + (jj / 4) * s.P) + (jj & 3);
-            uq[q] = u;
-            jq[q] = j;
-            const bool ok = i < n_work && j < H;
-            const int ul = s.lst[u], b = s.b[ul], cur = s.cur[ul];
+            const int k = i >> (lgn + 2), u = (i >> 2) & ((1 << lgn) - 1);
+            const int j = 4 * (redundant ? k : s.rank + k * s.P) + (i & 3);
+            const bool ok = i < n_work && u < nl;
+            const int ul = s.lst[u < nl ? u : 0], b = s.b[ul], old = s.cur[ul] ^ 1;
             const bool st = ok && !(s.flags[ul] & kFlagZeroHC);
             e[q] = ld4(B.ep, ok ? (unsigned)(((size_t)s.pend[ul] * 4 * H + 4 * j) * 4) : kBad);
-            r[q] = ld4_coh(B.rx, st ? (unsigned)((rx_off(p, cur, 0, b) + 4 * j) * 4) : kBad);
-            c_prev[q] = ld1_coh(B.cx, st ? (unsigned)((hx_off(p, cur, 0, b) + j) * 4) : kBad);
+            r[q] = ld4_coh(B.rx, st ? (unsigned)((rx_off(p, old, b) + 4 * j) * 4) : kBad);
+            c_prev[q] = ld1_coh(B.cx, st ? (unsigned)((cx_off(p, old, b) + j) * 4) : kBad);
         }
 #pragma unroll
         for (int q = 0; q < kL0; ++q) {
             const int i = base + threadIdx.x + q * kBlock;
-            const int u = uq[q], j = jq[q];
-            if (i >= n_work || j >= H) continue;
+            const int k = i >> (lgn + 2), u = (i >> 2) & ((1 << lgn) - 1), g = i & 3;
+            if (i >= n_work || u >= nl) continue;
+            const int tile = redundant ? k : s.rank + k * s.P, j = 4 * tile + g;
             const int ul = s.lst[u], b = s.b[ul], cur = s.cur[ul];
             float c_new, h_new;
             cell(e[q].x + r[q].x, e[q].y + r[q].y, e[q].z + r[q].z, e[q].w + r[q].w, c_prev[q], c_new, h_new);
             if (redundant) {   // straight into the layer-1 activation block
                 const Act &x = S.act[1];
                 split_f16(h_new, x.hi[u * x.kp + j], x.lo[u * x.kp + j]);
+            } else {
+                st_coh(p.hx + hx_at(p, s.dom, 0, half, tile, u) + g, filled(h_new));
             }
-            // owner of unit group j / 4 (always, when only this workgroup's units are listed)
-            if (!redundant || (j >> 2) - udiv(j >> 2, s.mag_p, s.P) * s.P == s.rank) {
-                st_coh(p.cx + hx_off(p, cur ^ 1, 0, b) + j, c_new);
-                st_coh(p.hx + hx_off(p, cur ^ 1, 0, b) + j, h_new);
+            // owner of the tile (always, when only this workgroup's units are listed)
+            if (!redundant || tile - udiv(tile, s.mag_p, s.P) * s.P == s.rank) {
+                st_coh(p.cx + cx_off(p, cur, b) + j, c_new);
+                st_coh(p.hs + hs_off(p, 0, b) + j, h_new);
             }
         }
     }
@@ -1458,7 +1494,7 @@ __device__ __forceinline__ void lstm_layer0(const KParams &p, Ctl &s, const Lds 
 //                    the four rows a lane holds are the four gates of one unit)
 //                    or W_p (pred projection) when lc is the last layer;
 //   recurrent tiles  W_hh_lc . h_lc' -> R_lc for the utterance's next step
-//                    (stored in the other ping-pong half of rx).
+//                    (R_0 in the half of rx of the new parity).
 // Column tile: utterances lst[c0 .. c0+nc).
 // Both matrices have K = H and the same storage type.
 // LDS state of layer l (>= 1), utterance ul, owned tile k.
@@ -1468,7 +1504,7 @@ __device__ __forceinline__ float *st_at(const KParams &p, const Lds &S, int l, i
 
 template <int WC>
 __device__ __forceinline__ void consume_layer(const KParams &p, Ctl &s, const Lds &S, const Bufs &B, const Act &x,
-                                              int lc, int c0, int nc) {
+                                              int lc, int half, int c0, int nc) {
     const int lane = threadIdx.x & (kWave - 1);
     const bool last = lc == p.L - 1;
     const TMat &wc = last ? p.w_pred : p.w_ih[lc + 1];
@@ -1493,7 +1529,7 @@ __device__ __forceinline__ void consume_layer(const KParams &p, Ctl &s, const Ld
                       const int k = it - n_c;
                       if (lc == 0) {        // R_0: read by the layer-0 update of every workgroup (global)
                           const int row0 = (s.rank + k * s.P) * kTile + g * 4;
-                          st4_coh(B.rx, (unsigned)((rx_off(p, cur ^ 1, 0, b) + row0) * 4),
+                          st4_coh(B.rx, (unsigned)((rx_off(p, cur, b) + row0) * 4),
                                   make_float4(acc[0], acc[1], acc[2], acc[3]));
                       } else {              // R_lc: LDS state of this workgroup
                           *reinterpret_cast<float4 *>(st_at(p, S, lc, ul, k) + g * 4) =
@@ -1503,9 +1539,12 @@ __device__ __forceinline__ void consume_layer(const KParams &p, Ctl &s, const Ld
                   }
                   const int row0 = (s.rank + it * s.P) * kTile + g * 4;
                   const float4 bias = *reinterpret_cast<const float4 *>(btab + it * kTile + g * 4);
-                  if (last) {               // pred projection: rows row0 .. row0+3 of pp
-                      st4_coh(B.ppx, (unsigned)(((size_t)b * p.J + row0) * 4),
-                              make_float4(acc[0] + bias.x, acc[1] + bias.y, acc[2] + bias.z, acc[3] + bias.w));
+                  if (last) {               // pred projection: rows row0 .. row0+3 of pp; the old ones emptied
+                      const int t = s.rank + it * s.P;
+                      st4_coh(B.ppx, (ppx_at(p, s.dom, cur, t, ul) + g * 4) * 4u,
+                              make_float4(filled(acc[0] + bias.x), filled(acc[1] + bias.y), filled(acc[2] + bias.z),
+                                          filled(acc[3] + bias.w)));
+                      st4_coh(B.ppx, (ppx_at(p, s.dom, cur ^ 1, t, ul) + g * 4) * 4u, empty4());
                       return;
                   }
                   // cell update of unit j = row0 / 4 of layer `layer`: R and c_prev from the LDS state
@@ -1520,136 +1559,128 @@ __device__ __forceinline__ void consume_layer(const KParams &p, Ctl &s, const Ld
                   cell((acc[0] + r.x) + bias.x, (acc[1] + r.y) + bias.y, (acc[2] + r.z) + bias.z,
                        (acc[3] + r.w) + bias.w, c_prev, c_new, h_new);
                   st[kTile + g] = c_new;
-                  st_coh(p.hx + hx_off(p, cur ^ 1, layer, b) + row0 / 4, h_new);
+                  st_coh(p.hx + hx_at(p, s.dom, layer, half, s.rank + it * s.P, c0 + u) + g, filled(h_new));
+                  st_coh(p.hs + hs_off(p, layer, b) + row0 / 4, h_new);
               });
+}
+
+// Empty this workgroup's tiles of h (every layer) in one half of hx, rows below n.
+__device__ __forceinline__ void empty_h(const KParams &p, const Ctl &s, const Bufs &B, int half, int n) {
+    const int lr = __builtin_ctz((unsigned)p.rows), per = s.own_lstm << lr;
+    for (int l = p.hl0; l < p.L; ++l)
+        for (int i = threadIdx.x; i < per; i += kBlock) {
+            const int u = i & (p.rows - 1), t = s.rank + (i >> lr) * s.P;
+            if (u < n) st4_coh(B.hx, hx_at(p, s.dom, l, half, t, u) * 4u, empty4());
+        }
 }
 
 // One LSTM step (all layers), the pred projection and the recurrent products
 // for every utterance of the LSTM list.  A small list in a whole-device
-// domain runs layer 0 redundantly in every workgroup (no barrier between
-// layers 0 and 1); otherwise layer 0 is split by unit tiles and followed by a
-// barrier.  Each later phase stages one layer's full new output and runs the
-// tiles that consume it.
+// domain runs layer 0 redundantly in every workgroup (no exchange between
+// layers 0 and 1); otherwise layer 0 is split by unit tiles.  Each later phase
+// stages one layer's full new output as it arrives and runs the tiles that
+// consume it.  half: the half of hx this step uses; n_prev: list length of the
+// previous step, whose half is emptied here.
 template <int WC>
-__device__ __forceinline__ bool lstm_and_pred(const KParams &p, Ctl &s, const Bufs &B, const Lds &S, unsigned &epoch,
-                              unsigned long long &tlast) {
-    const int H = p.H, L = p.L;
+__device__ __forceinline__ void lstm_and_pred(const KParams &p, Ctl &s, const Bufs &B, const Lds &S, int half,
+                                              int n_prev, unsigned long long &tlast) {
+    const int L = p.L;
     const bool redundant = s.nl <= kSmallB && p.n_dom == 1;
-    lstm_layer0(p, s, S, B, redundant);
+    lstm_layer0(p, s, S, B, redundant, half);
+    empty_h(p, s, B, half ^ 1, n_prev);
     TLA(1);
     pmark(p, s, tlast, kPrL0);
     for (int lc = 0; lc < L; ++lc) {
         const bool local = lc == 0 && redundant;     // h_0' is in LDS already
-        if (!local) {
-            if (!dom_sync(p, s, epoch)) return false;
-            TLA(18 + lc);
-            pmark(p, s, tlast, lc == 0 ? kPrSync0 : kPrSync1);
-        }
         for (int c0 = 0; c0 < s.nl; c0 += kTile) {
             const int nc = min(kTile, s.nl - c0);
             Act x = S.act[1];
             x.n = nc;
-            if (!local) {   // (redundant layer 0 wrote h_0' into the block itself)
-                stage_act(x, H, nc, B.hx, [&](int u) { const int ul = s.lst[c0 + u]; return hx_off(p, s.cur[ul] ^ 1, lc, s.b[ul]); });
-            }
+            // (redundant layer 0 wrote h_0' into the block itself.)  The block's last readers, the
+            // previous products, are behind the barrier that opens their reduce.
+            if (!local) stage_h(p, s, B, x, lc, half, c0, nc);
             TLBASE(2 + 8 * lc);
             lds_sync();
             TL(0);
-            pmark(p, s, tlast, kPrStageL);
-            consume_layer<WC>(p, s, S, B, x, lc, c0, nc);
+            pmark(p, s, tlast, lc == 0 ? kPrStage0 : kPrStage1);
+            consume_layer<WC>(p, s, S, B, x, lc, half, c0, nc);
             TL(6);
         }
         pmark(p, s, tlast, lc == L - 1 ? kPrPred : kPrL1);
     }
-    for (int i = threadIdx.x; i < s.nl; i += kBlock) {   // the new state becomes current
+    for (int i = threadIdx.x; i < s.nl; i += kBlock) {   // the step is taken
         const int ul = s.lst[i];
-        s.cur[ul] ^= 1;
         s.pend[ul] = -1;
         s.flags[ul] &= ~kFlagZeroHC;
+        s.stp[ul] = 1;
     }
-    const bool ok = dom_sync(p, s, epoch);
-    TLA(20);
-    pmark(p, s, tlast, kPrSync2);
-    return ok;
 }
 
 // Apply the argmax results of iteration `stamp` to every utterance of the joint
 // list: src/parakeet_tdt.cpp:936-967 (TDT) and src/parakeet_eou.cpp:275-332 (EOU).
-// The domain's best key per joint column and head: the maximum over the
-// shards that carry this iteration's stamp (shards no rank wrote this
-// iteration hold older stamps and are skipped).  Lane groups of p.shards
-// reduce one (column, head) with shuffles; results go to s.wgkey.
-__device__ __forceinline__ void gather_shards(const KParams &p, Ctl &s, unsigned stamp) {
-    const int G = p.shards, lg = __builtin_ctz((unsigned)G);   // a power of two
-    const unsigned long long *keys = p.keys + (size_t)(stamp & 1) * p.n_dom * kColCap * G * 2;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int n = s.ncol * 2 * G;
-    for (int e0 = 0; e0 < n; e0 += kBlock) {      // e = (pair, shard); whole waves stay together
-        const int e = e0 + threadIdx.x;
-        unsigned long long k = 0ull;
-        if (e < n) {
-            const int pair = e >> lg, sh = e & (G - 1);
-            const size_t col = (size_t)s.dom * kColCap + (pair >> 1);
-            k = __hip_atomic_load(&keys[(col * G + sh) * 2 + (pair & 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (key_stamp(k) != stamp) k = 0ull;
-        }
-        for (int m = 1; m < G; m <<= 1) {
-            const unsigned long long o = __shfl_xor(k, m, kWave);
-            k = o > k ? o : k;
-        }
-        if (e < n && (lane & (G - 1)) == 0) {
-            const int pair = e >> lg;
-            s.wgkey[pair >> 1][pair & 1] = k;
-        }
-    }
-    lds_sync();
-}
-
-// The domain's best key per joint column and head from the workgroups' slots
-// (slot mode): thread e polls slot (pair e / P, rank e % P) until it carries
-// stamp, each wave takes the maximum per pair, and one LDS atomic max per wave
-// and pair lands in s.wgkey (stamped keys are above the unstamped local ones it
-// holds).  Bounded like dom_sync: false on an error or a ~2 s wait.
-__device__ __forceinline__ bool gather_slots(const KParams &p, Ctl &s, unsigned stamp) {
-    __shared__ int s_ok;
-    if (threadIdx.x == 0) s_ok = 1;
-    lds_sync();   // this workgroup's slot stores have read s.wgkey
-    const int P = s.P, npair = 2 * s.ncol, n = npair * P;
-    const unsigned long long *sl = p.slots + (size_t)(stamp & 1) * P * kSlotCols * 2;
-    const int lane = threadIdx.x & (kWave - 1);
-    for (int e0 = 0; e0 < n; e0 += kBlock) {   // whole waves stay together
-        const int e = e0 + threadIdx.x;
-        unsigned long long k = 0ull;
-        int pair = -1;
-        if (e < n) {
-            pair = udiv(e, s.mag_p, P);
-            const int r = e - pair * P;
-            const unsigned long long *w = sl + ((size_t)r * kSlotCols + (pair >> 1)) * 2 + (pair & 1);
-            const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-            unsigned m = 0;
-            while (key_stamp(k = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != stamp) {
-                if ((++m & 63) != 0) continue;
-                if (__hip_atomic_load(p.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) { s_ok = 0; break; }
-                if (__builtin_amdgcn_s_memrealtime() - t0 > 200000000ull) {   // 100 MHz clock: 2 s
-                    __hip_atomic_store(p.status, PK_ERR_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    s_ok = 0;
-                    break;
-                }
-            }
-        }
-        for (int q = 0; q < npair; ++q) {
-            unsigned long long v = pair == q ? k : 0ull;
+// The domain's best key per joint column and head.  Token keys: lane groups of
+// `pairs` threads load two columns of one rank each (16 bytes) until both carry
+// this iteration's stamp, every rank of the domain; then the wave's maximum per
+// column and one LDS atomic max per wave.  Duration keys come from the ranks that
+// own duration rows.  The stamp is the arrival signal: a workgroup that has seen
+// every rank's keys knows that all of them are done with the iteration's staged
+// data.  A rank cannot overwrite a key before every workgroup has read it: it
+// stores the same half again two iterations on, after the keys of the next.
+constexpr int kKeyRounds = 4;
+__device__ __forceinline__ void gather_keys(const KParams &p, Ctl &s, const Bufs &B, unsigned stamp) {
+    lds_sync();   // this workgroup's key stores have read s.wgkey
+    const int P = s.P, nc = s.ncol, lane = threadIdx.x & (kWave - 1);
+    const int lgp = nc <= 2 ? 0 : 31 - __builtin_clz((unsigned)(nc - 1));   // log2 of the column pairs, rounded up
+    const int pairs = 1 << lgp, cp = threadIdx.x & (pairs - 1), r0 = threadIdx.x >> lgp, step = kBlock >> lgp;
+    const unsigned dom = (stamp & 1) * p.n_dom + s.dom;
+    const unsigned base = (dom * P * p.cols + 2 * cp) * 8u, stride = (unsigned)p.cols * 8u;
+    const bool two = 2 * cp + 1 < nc, one = 2 * cp < nc;
+    // the duration word of this thread, polled with its first round
+    const int lc = __builtin_ctz((unsigned)p.cols), dc = threadIdx.x & (p.cols - 1), dd = threadIdx.x >> lc;
+    bool want_d = dd < p.n_durk && dc < nc;
+    const unsigned doff = (2u * p.n_dom * P * p.cols + (dom * 2 + dd) * p.cols + dc) * 8u;
+    unsigned long long best0 = 0ull, best1 = 0ull, kd = 0ull;
+    for (int rb = 0; rb < P; rb += step * kKeyRounds) {
+        unsigned pend = 0u, n = 0u;
+        unsigned long long since = 0ull;
 #pragma unroll
-            for (int m = 1; m < kWave; m <<= 1) {
-                const unsigned long long o = __shfl_xor(v, m, kWave);
-                v = o > v ? o : v;
+        for (int q = 0; q < kKeyRounds; ++q)
+            if (one && rb + r0 + step * q < P) pend |= 1u << q;
+        while (pend != 0u || want_d) {
+            typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
+            u64x2 v[kKeyRounds];
+#pragma unroll
+            for (int q = 0; q < kKeyRounds; ++q)
+                v[q] = __builtin_bit_cast(u64x2, ld4_coh(B.keys, (pend >> q) & 1u
+                                                                     ? base + (unsigned)(rb + r0 + step * q) * stride
+                                                                     : kBad));
+            const unsigned long long d = __builtin_bit_cast(
+                unsigned long long, __builtin_amdgcn_raw_buffer_load_b64(B.keys, want_d ? doff : kBad, 0, kSC1));
+#pragma unroll
+            for (int q = 0; q < kKeyRounds; ++q)
+                if (((pend >> q) & 1u) && key_stamp(v[q][0]) == stamp && (!two || key_stamp(v[q][1]) == stamp)) {
+                    best0 = v[q][0] > best0 ? v[q][0] : best0;
+                    best1 = two && v[q][1] > best1 ? v[q][1] : best1;
+                    pend &= ~(1u << q);
+                }
+            if (want_d && key_stamp(d) == stamp) {
+                kd = d;
+                want_d = false;
             }
-            if (lane == 0 && v != 0ull) atomicMax(&s.wgkey[q >> 1][q & 1], v);
+            if ((pend != 0u || want_d) && wait_over(p, s, n, since)) break;
         }
     }
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    if (kd != 0ull) atomicMax(&s.wgkey[dc][1], kd);
+    for (int m = pairs; m < kWave; m <<= 1) {
+        const unsigned long long o0 = __shfl_xor(best0, m, kWave), o1 = __shfl_xor(best1, m, kWave);
+        best0 = o0 > best0 ? o0 : best0;
+        best1 = o1 > best1 ? o1 : best1;
+    }
+    if (lane < pairs) {
+        if (best0 != 0ull) atomicMax(&s.wgkey[2 * cp][0], best0);
+        if (best1 != 0ull) atomicMax(&s.wgkey[2 * cp + 1][0], best1);
+    }
     lds_sync();
-    return s_ok != 0;
 }
 
 // One utterance per thread.  Its first decision is column i (frame t); while
@@ -1704,6 +1735,7 @@ __device__ __forceinline__ void decide_steps(const KParams &p, Ctl &s, unsigned 
                         else s.flags[ul] |= kFlagTokOverflow;
                     }
                     s.pend[ul] = tok;
+                    s.cur[ul] ^= 1;
                     s.sym[ul] += 1;
                     if (dur > 0 || s.sym[ul] >= p.max_sym) {
                         s.t[ul] += adv;
@@ -1728,6 +1760,7 @@ __device__ __forceinline__ void decide_steps(const KParams &p, Ctl &s, unsigned 
                     }
                     s.flags[ul] |= kFlagZeroHC;
                     s.pend[ul] = p.blank;
+                    s.cur[ul] ^= 1;
                     s.last[ul] = p.blank;
                     frame_done = true;
                 } else if (tok >= 0 && tok < p.n_special && p.special[tok]) {
@@ -1740,6 +1773,7 @@ __device__ __forceinline__ void decide_steps(const KParams &p, Ctl &s, unsigned 
                         else s.flags[ul] |= kFlagTokOverflow;
                     }
                     s.pend[ul] = tok;
+                    s.cur[ul] ^= 1;
                     s.last[ul] = tok;
                     s.sym[ul] += 1;
                     if (s.sym[ul] >= max_syms) frame_done = true;
@@ -1777,9 +1811,7 @@ __device__ __forceinline__ void tap_copy(const KParams &p, Ctl &s) {
     if (threadIdx.x == 0) s.tq_n = 0;
 }
 
-__device__ __forceinline__ void decide(const KParams &p, Ctl &s, unsigned stamp, bool gathered) {
-    if (!gathered) gather_shards(p, s, stamp);
-    TLA(30);
+__device__ __forceinline__ void decide(const KParams &p, Ctl &s, unsigned stamp) {
     if (s.ncol > s.nj) decide_steps<true>(p, s, stamp);
     else decide_steps<false>(p, s, stamp);
     if (p.logits) tap_copy(p, s);
@@ -1841,7 +1873,7 @@ __device__ __forceinline__ bool coresident(const KParams &p) {
     return s_dec == kArriveGo;
 }
 
-template <int WC, bool ONE>
+template <int WC>
 __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     __shared__ Ctl s;
@@ -1850,10 +1882,11 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
     const int H = p.H, L = p.L, J = p.J, n_all = p.n_utts;
     unsigned epoch = 0;
     Bufs B;
-    B.hx = rsrc(p.hx, (unsigned)((size_t)2 * L * n_all * H * 4));
-    B.cx = rsrc(p.cx, (unsigned)((size_t)2 * L * n_all * H * 4));
-    B.ppx = rsrc(p.ppx, (unsigned)((size_t)n_all * J * 4));
-    B.rx = rsrc(p.rx, (unsigned)((size_t)2 * L * n_all * 4 * H * 4));
+    B.hx = rsrc(p.hx, (unsigned)((size_t)2 * (L - p.hl0) * p.n_dom * H * p.rows * 4));
+    B.cx = rsrc(p.cx, (unsigned)((size_t)2 * n_all * H * 4));
+    B.ppx = rsrc(p.ppx, (unsigned)((size_t)2 * p.n_dom * J * p.prows * 4));
+    B.rx = rsrc(p.rx, (unsigned)((size_t)2 * n_all * 4 * H * 4));
+    B.keys = rsrc(p.keys, (unsigned)((size_t)2 * p.n_dom * (p.dom_size + 2) * p.cols * 8));
     B.ep = rsrc(p.eproj, (unsigned)((size_t)p.V1 * 4 * H * 4));
     B.encp = rsrc(p.encp, (unsigned)(p.encp_rows * J * 4));
 
@@ -1901,8 +1934,7 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
             s.pass[lc] = p.red_slots / units_per_item(lc == p.L - 1 ? p.w_pred : p.w_ih[lc + 1]);
         s.pass[p.L] = p.red_slots / units_per_item(p.w_out);
         s.mag_p = udiv_magic(s.P);
-        s.mag_h = udiv_magic(p.H);
-        s.mag_units = udiv_magic(4 * s.own_lstm);
+        s.ok = 1;
         unsigned wm = 0;
         for (int ul = 0; ul < kDomCap; ++ul) wm |= (ul % s.P == s.rank ? 1u : 0u) << ul;
         s.wmask = wm;
@@ -1922,7 +1954,8 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
         s.ntok[ul] = 0;
         s.steps[ul] = 0;
         s.nseg[ul] = 0;
-        s.cur[ul] = 0;
+        s.cur[ul] = init ? 0 : 1;   // (a fresh utterance's first step is pending)
+        s.stp[ul] = 0;
         s.sym[ul] = init ? ctrl[PK_CTRL_SYM] : 0;
         if (p.kind == PK_KIND_EOU && s.T[ul] > 0) s.sym[ul] = 0;   // reset per frame (src/parakeet_eou.cpp:269)
         s.last[ul] = init ? ctrl[PK_CTRL_LAST] : -1;
@@ -1935,29 +1968,37 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
         else s.t[ul] = 0;
     }
     __syncthreads();
-    // copy the slot state of this workgroup's utterances into the exchange
-    // buffers (kCopyB loads in flight per thread, then the stores)
-    const __amdgpu_buffer_rsrc_t bx = rsrc(p.hx, p.xchg_bytes);
-    const int nq = state_chunks(p);
+    // copy c_0, R_0 and pp of this workgroup's utterances from their slots into the
+    // exchange buffers (kCopyB loads in flight per thread, then the stores), and empty
+    // the words the loop waits for: the other half of pp, this workgroup's tiles of h
     for (int ul = s.rank; ul < s.n; ul += s.P) {
         const int b = s.b[ul], slot = p.slot[b];
+        const bool fresh = s.flags[ul] & kFlagZeroHC;
+        const float *src_c = p.slot_c + (size_t)slot * L * H, *src_r = p.slot_r + (size_t)slot * L * 4 * H,
+                    *src_p = p.slot_pp + (size_t)slot * J;
+        const int nq = fresh ? 0 : (H + 4 * H + J) / 4;
         for (int q0 = 0; q0 < nq; q0 += kCopyB * kBlock) {
             float4 v[kCopyB];
-            long long xo[kCopyB];
 #pragma unroll
             for (int j = 0; j < kCopyB; ++j) {
-                const int q = q0 + threadIdx.x + j * kBlock;
-                if (q < nq) {
-                    const StateChunk c = state_chunk(p, q, slot, b, 0);
-                    v[j] = *reinterpret_cast<const float4 *>(c.slot);
-                    xo[j] = c.x;
-                }
+                const int i = 4 * min(q0 + (int)threadIdx.x + j * kBlock, nq - 1);
+                v[j] = *reinterpret_cast<const float4 *>(i < H ? src_c + i : i < 5 * H ? src_r + (i - H) : src_p + (i - 5 * H));
             }
 #pragma unroll
-            for (int j = 0; j < kCopyB; ++j)
-                if (q0 + threadIdx.x + j * kBlock < nq) st4_coh(bx, (unsigned)(xo[j] * 4), v[j]);
+            for (int j = 0; j < kCopyB; ++j) {
+                const int q = q0 + threadIdx.x + j * kBlock, i = 4 * q;
+                if (q >= nq) continue;
+                if (i < H) st4_coh(B.cx, (unsigned)((cx_off(p, 0, b) + i) * 4), v[j]);
+                else if (i < 5 * H) st4_coh(B.rx, (unsigned)((rx_off(p, 0, b) + (i - H)) * 4), v[j]);
+                else st4_coh(B.ppx, (ppx_at(p, s.dom, 0, (i - 5 * H) / kTile, ul) + (i - 5 * H) % kTile) * 4u,
+                             make_float4(filled(v[j].x), filled(v[j].y), filled(v[j].z), filled(v[j].w)));
+            }
         }
+        for (int i = 4 * threadIdx.x; i < J; i += 4 * kBlock)
+            st4_coh(B.ppx, (ppx_at(p, s.dom, 1, i / kTile, ul) + i % kTile) * 4u, empty4());
     }
+    empty_h(p, s, B, 0, s.n);
+    empty_h(p, s, B, 1, s.n);
     bias_table(p, s.rank, s.P, S.bias);
     // LDS state of layers >= 1: R and c of this workgroup's unit tiles for every utterance of the domain
     if (L > 1) {
@@ -1981,6 +2022,7 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
     bool ok = dom_sync(p, s, epoch);
 
     unsigned iter = 0;
+    int half = 0, n_prev = 0;   // half of hx of the next LSTM step; list length of the previous one
     unsigned long long tlast = __builtin_amdgcn_s_memrealtime();
     while (ok) {
         if (s.nl == 0 && s.nj == 0) break;
@@ -2003,17 +2045,20 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
         float4 epre[kStageMax];
         if (s.nj > 0) encp_prefetch(p, s, B, epre);
         if (s.nl > 0) {
-            ok = lstm_and_pred<WC>(p, s, B, S, epoch, tlast);
-            if (!ok) break;
+            lstm_and_pred<WC>(p, s, B, S, half, n_prev, tlast);
+            half ^= 1;
+            n_prev = s.nl;
         }
         if (s.nj > 0) {
-            joint_phase<WC, ONE>(p, s, B, S, iter, epre, tlast);
-            const bool slots = slot_mode<ONE>(s);
-            ok = slots ? gather_slots(p, s, iter) : dom_sync(p, s, epoch);
+            joint_phase<WC>(p, s, B, S, iter, epre, tlast);
+            gather_keys(p, s, B, iter);
             TLA(29);
-            pmark(p, s, tlast, kPrJSync);
-            if (!ok) break;
-            decide(p, s, iter, slots);
+            pmark(p, s, tlast, kPrKeys);
+            if (!s.ok) {   // (behind the gather's barrier: the same in every wave)
+                ok = false;
+                break;
+            }
+            decide(p, s, iter);
         }
         lds_sync();
         build_lists(s, p.spec != 0);
@@ -2025,7 +2070,9 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
     if (p.prof && wg == 0 && threadIdx.x < kWaves * kTl) p.prof[kPrN + threadIdx.x] = tl_sum()[threadIdx.x];
     if (p.prof && wg == 0 && threadIdx.x < kTl) p.prof[kPrN + kWaves * kTl + threadIdx.x] = tl_ctl()[2 + threadIdx.x];
 #endif
-    if (!ok) return;
+    __builtin_amdgcn_s_waitcnt(0);   // this workgroup's state stores have landed
+    __syncthreads();
+    if (!ok || !s.ok) return;
 
     if (L > 1) {       // layers >= 1: R and c of this workgroup's unit tiles, from its LDS state
         const int n_own = owned(p.w_hh[1].tiles, s.rank, s.P);
@@ -2039,23 +2086,41 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
             else p.slot_c[((size_t)slot * L + l) * H + t * 4 + (e - kTile)] = v;
         }
     }
+    // h of every layer, c_0, R_0 and pp of this workgroup's tiles, for the utterances that took a
+    // step (the others' slots hold them already)
+    {
+        const __amdgpu_buffer_rsrc_t bx = rsrc(p.hs, p.xchg_bytes);
+        const int per = L + 1 + 4, n1 = s.n * s.own_lstm * per, n2 = s.n * s.own_pred * 4;
+        for (int i = threadIdx.x; i < n1 + n2; i += kBlock) {
+            float *dst;
+            long long x;   // float offset from p.hs
+            int ul;
+            if (i < n1) {
+                const int e = i % per, k = (i / per) % s.own_lstm, j = 4 * (s.rank + k * s.P);
+                ul = i / per / s.own_lstm;
+                const int b = s.b[ul], slot = p.slot[b], cur = s.cur[ul];
+                if (e < L) {
+                    dst = p.slot_h + ((size_t)slot * L + e) * H + j;
+                    x = (long long)hs_off(p, e, b) + j;
+                } else if (e == L) {
+                    dst = p.slot_c + (size_t)slot * L * H + j;
+                    x = (p.cx - p.hs) + (long long)cx_off(p, cur, b) + j;
+                } else {
+                    const int row = 4 * j + 4 * (e - L - 1);
+                    dst = p.slot_r + (size_t)slot * L * 4 * H + row;
+                    x = (p.rx - p.hs) + (long long)rx_off(p, cur, b) + row;
+                }
+            } else {
+                const int q = i - n1, g = q & 3, k = (q >> 2) % s.own_pred, t = s.rank + k * s.P;
+                ul = (q >> 2) / s.own_pred;
+                dst = p.slot_pp + (size_t)p.slot[s.b[ul]] * J + t * kTile + g * 4;
+                x = (p.ppx - p.hs) + (long long)ppx_at(p, s.dom, s.cur[ul], t, ul) + g * 4;
+            }
+            if (s.stp[ul]) *reinterpret_cast<float4 *>(dst) = ld4_coh(bx, (unsigned)(x * 4));
+        }
+    }
     for (int ul = s.rank; ul < s.n; ul += s.P) {
         const int b = s.b[ul], slot = p.slot[b];
-        const int cur = s.cur[ul];
-        for (int q0 = 0; q0 < nq; q0 += kCopyB * kBlock) {
-            float4 v[kCopyB];
-            float *dst[kCopyB];
-#pragma unroll
-            for (int j = 0; j < kCopyB; ++j) {
-                const int q = q0 + threadIdx.x + j * kBlock;
-                const StateChunk c = state_chunk(p, min(q, nq - 1), slot, b, cur);
-                v[j] = ld4_coh(bx, q < nq ? (unsigned)(c.x * 4) : kBad);
-                dst[j] = c.slot;
-            }
-#pragma unroll
-            for (int j = 0; j < kCopyB; ++j)
-                if (q0 + threadIdx.x + j * kBlock < nq) *reinterpret_cast<float4 *>(dst[j]) = v[j];
-        }
         if (threadIdx.x < PK_CTRL_N) {   // the slot's control words (and the caller's copy)
             const int k = threadIdx.x;
             const int v = k == PK_CTRL_INIT ? 1
