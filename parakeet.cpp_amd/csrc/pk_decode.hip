@@ -8,8 +8,8 @@
 //                       once per window (src/parakeet_tdt.cpp:433-483 computes
 //                       the same projection as a ggml graph; the CPU path
 //                       recomputes it per step at :167-168).  At most
-//                       kNarrowRows rows: enc_proj_narrow_kernel instead
-//                       (bit-identical outputs).
+//                       kNarrowRows rows: enc_proj_narrow_kernel, at least
+//                       kWideRows: enc_proj_wide_kernel (bit-identical outputs).
 //   decode_loop_kernel  all lockstep iterations of all utterances in one
 //                       launch (an ordinary dispatch whose workgroups first
 //                       check that the whole grid is resident, relaunched
@@ -84,6 +84,10 @@ constexpr int kCacheMinFrames = 16;
 // enc_proj over at most this many rows runs the narrow kernel (one wave per 16x16 block;
 // measured faster up to 256 rows, slower from 750 on)
 constexpr long long kNarrowRows = 256;
+// enc_proj over at least this many rows runs the wide kernel (128 x 320 tiles; measured against the
+// 64 x 64 tiles with q8_0, f16 and f32 weights: 8,192 rows 51 / 55 us, 46 / 51, 61 / 66; 16,384 rows
+// 94 / 59, 87 / 56, 112 / 73)
+constexpr long long kWideRows = 10240;
 
 thread_local std::string g_err;
 
@@ -378,7 +382,9 @@ int scratch_address(int device, unsigned char **out) {
 struct pk_decoder {
     KParams kp{};              // weights + dims (batch fields filled per call)
     pk_decoder_desc desc{};    // host copy of the description (tensor pointers not kept)
-    const _Float16 *w_enc_hi = nullptr, *w_enc_lo = nullptr;   // joint.enc [J][D] as f16 hi + lo planes
+    int enc_w = 0;                                              // joint.enc storage (pkdev::kEp*)
+    const _Float16 *w_enc_hi = nullptr, *w_enc_lo = nullptr;   // joint.enc [J][D] (see pkdev::EncProj)
+    const float *w_enc_scale = nullptr;                         // joint.enc block scales [D/32][J]
     const float *b_enc = nullptr;                               // joint.enc bias
     int n_slots = 0;
     int device = 0;
@@ -641,19 +647,42 @@ PK_API int pk_decoder_create(const pk_decoder_desc *d, int32_t n_slots, pk_decod
     if ((rc = vec_f32(d->joint_pred_b, J, nullptr, b_pred, "joint.pred.bias"))) return cleanup(rc);
     if ((rc = vec_f32(d->joint_out_b, Vo, nullptr, b_out, "joint.out.bias"))) return cleanup(rc);
     if ((rc = vec_f32(d->joint_enc_b, J, nullptr, b_enc, "joint.enc.bias"))) return cleanup(rc);
-    if ((rc = dense_f32(d->joint_enc_w, J, D, nullptr, w_enc, "joint.enc.weight"))) return cleanup(rc);
+    if ((rc = check_tensor(d->joint_enc_w, J, D, "joint.enc.weight"))) return cleanup(rc);
     // joint.out bias padded with zeros to whole 16-row tiles (read a float4 per lane)
     b_out.resize((size_t)(Vo + kTile - 1) / kTile * kTile, 0.0f);
     ar.add(b_pred.data(), b_pred.size() * 4, reinterpret_cast<const void **>(&kp.b_pred));
     ar.add(b_out.data(), b_out.size() * 4, reinterpret_cast<const void **>(&kp.b_out));
     ar.add(b_enc.data(), b_enc.size() * 4, reinterpret_cast<const void **>(&dec->b_enc));
-    std::vector<_Float16> w_enc_hi(w_enc.size()), w_enc_lo(w_enc.size());
-    for (size_t i = 0; i < w_enc.size(); ++i) {
-        w_enc_hi[i] = (_Float16)w_enc[i];
-        w_enc_lo[i] = (_Float16)(w_enc[i] - (float)w_enc_hi[i]);
+    std::vector<_Float16> w_enc_hi((size_t)J * D), w_enc_lo;
+    std::vector<float> w_enc_scale;
+    if (quantized(d->joint_enc_w.type)) {   // exact integers, f32 block scales by K block
+        dec->enc_w = pkdev::kEpQuant;
+        w_enc_scale.resize((size_t)J * (D / 32));
+        const int bb = block_bytes(d->joint_enc_w.type);
+        const uint8_t *blk = static_cast<const uint8_t *>(d->joint_enc_w.data);
+        for (int j = 0; j < J; ++j)
+            for (int kb = 0; kb < D / 32; ++kb, blk += bb) {
+                uint16_t dh;
+                int8_t q[32];
+                block_q(blk, d->joint_enc_w.type, dh, q);
+                w_enc_scale[(size_t)kb * J + j] = f16_to_f32(dh);
+                for (int i = 0; i < 32; ++i) w_enc_hi[(size_t)j * D + kb * 32 + i] = (_Float16)(float)q[i];
+            }
+    } else {                                // f16 as stored; f32 as hi + lo
+        const bool full = d->joint_enc_w.type != PK_TYPE_F16;
+        dec->enc_w = full ? pkdev::kEpFull : pkdev::kEpHalf;
+        if ((rc = dense_f32(d->joint_enc_w, J, D, nullptr, w_enc, "joint.enc.weight"))) return cleanup(rc);
+        if (full) w_enc_lo.resize(w_enc.size());
+        for (size_t i = 0; i < w_enc.size(); ++i) {
+            w_enc_hi[i] = (_Float16)w_enc[i];
+            if (full) w_enc_lo[i] = (_Float16)(w_enc[i] - (float)w_enc_hi[i]);
+        }
     }
     ar.add(w_enc_hi.data(), w_enc_hi.size() * 2, reinterpret_cast<const void **>(&dec->w_enc_hi));
-    ar.add(w_enc_lo.data(), w_enc_lo.size() * 2, reinterpret_cast<const void **>(&dec->w_enc_lo));
+    if (!w_enc_lo.empty())
+        ar.add(w_enc_lo.data(), w_enc_lo.size() * 2, reinterpret_cast<const void **>(&dec->w_enc_lo));
+    if (!w_enc_scale.empty())
+        ar.add(w_enc_scale.data(), w_enc_scale.size() * 4, reinterpret_cast<const void **>(&dec->w_enc_scale));
     if ((rc = ar.upload(dec->arena))) return cleanup(rc);
     // f32 matrices: the lo plane follows the hi plane in the same upload
     {
@@ -1122,6 +1151,26 @@ int after_not_resident(pk_decoder *dec, int *d_status) {
     return 0;
 }
 
+template <int W>
+void launch_enc_proj(char which, const pkdev::EncProj &e, hipStream_t st) {
+    if (which == 'n') {
+        pkdev::enc_proj_narrow_kernel<W><<<dim3((unsigned)((e.rows + 15) / 16), 1, (e.J + 63) / 64), 256, 0, st>>>(e);
+    } else if (which == 'w') {
+        const long long blocks = (e.rows + pkdev::kEwRows - 1) / pkdev::kEwRows;
+        const int n_col = (e.J + pkdev::kEwCols - 1) / pkdev::kEwCols;
+        pkdev::enc_proj_wide_kernel<W><<<(unsigned)((blocks + 7) / 8 * 8 * n_col), pkdev::kEwThreads, 0, st>>>(e);
+    } else {
+        const dim3 grid((unsigned)((e.rows + pkdev::kEpTile - 1) / pkdev::kEpTile), 1,
+                        (e.J + pkdev::kEpTile - 1) / pkdev::kEpTile);
+        pkdev::enc_proj_kernel<W><<<grid, 256, 0, st>>>(e);
+    }
+}
+void launch_enc_proj(int w, char which, const pkdev::EncProj &e, hipStream_t st) {
+    if (w == pkdev::kEpQuant) launch_enc_proj<pkdev::kEpQuant>(which, e, st);
+    else if (w == pkdev::kEpHalf) launch_enc_proj<pkdev::kEpHalf>(which, e, st);
+    else launch_enc_proj<pkdev::kEpFull>(which, e, st);
+}
+
 int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratch cs) {
     if (!dec || !bt) return fail(PK_ERR_ARG, "pk_decode: null argument");
     dec->chained = false;   // (decode_chained sets it again after its last launch)
@@ -1292,22 +1341,12 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
     if (rows > 0) {
         if ((rc = cs.get(dec->d_encp, (size_t)rows * J * 4, reinterpret_cast<void **>(&d_encp)))) return rc;
         // tiles over the packed rows of all utterances; the kernel also clears the loop's words.
-        // Both kernels give bit-identical rows (PK_ENC_PROJ=tile / narrow forces one).
+        // The kernels give bit-identical rows (PK_ENC_PROJ=narrow / tile / wide forces one).
         const char *ep_env = std::getenv("PK_ENC_PROJ");
-        const bool narrow = ep_env ? ep_env[0] == 'n' : rows <= kNarrowRows;
-        if (narrow) {
-            dim3 grid((unsigned)((rows + 15) / 16), 1, (J + 63) / 64);
-            pkdev::enc_proj_narrow_kernel<<<grid, 256, 0, dec->stream>>>(dec->w_enc_hi, dec->w_enc_lo, J, dec->b_enc,
-                                                                         enc, D, d_src, d_dst, m, rows, d_encp,
-                                                                         static_cast<unsigned *>(d_clear),
-                                                                         clear_words);
-        } else {
-            dim3 grid((unsigned)((rows + pkdev::kEpTile - 1) / pkdev::kEpTile), 1,
-                      (J + pkdev::kEpTile - 1) / pkdev::kEpTile);
-            pkdev::enc_proj_kernel<<<grid, 256, 0, dec->stream>>>(dec->w_enc_hi, dec->w_enc_lo, J, dec->b_enc, enc,
-                                                                  D, d_src, d_dst, m, rows, d_encp,
-                                                                  static_cast<unsigned *>(d_clear), clear_words);
-        }
+        const char which = ep_env ? ep_env[0] : rows <= kNarrowRows ? 'n' : rows < kWideRows ? 't' : 'w';
+        pkdev::EncProj ep{dec->w_enc_hi, dec->w_enc_lo, dec->w_enc_scale, dec->b_enc, enc, J, D, m, d_src, d_dst, rows,
+                          d_encp, static_cast<unsigned *>(d_clear), clear_words};
+        launch_enc_proj(dec->enc_w, which, ep, dec->stream);
         HIP_TRY(hipGetLastError());
     } else {
         pkdev::fill_zero_kernel<<<(unsigned)std::min<size_t>((clear_words + 255) / 256, 1024), 256, 0, dec->stream>>>(

@@ -340,167 +340,284 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(unsigned *__restrict p, 
 // ---------------------------------------------------------------- enc_proj
 
 // encp[rows of utterance u] = b_e + W_e . enc[row] for every frame: an MFMA
-// GEMM with f32 accuracy.  Frames (f32) are split into f16 hi + lo when staged
-// in LDS; W_e arrives as f16 hi / lo planes [J][D] (split once at load).
-// Each 16x16 output tile takes hi.hi + lo.hi + hi.lo (the lo.lo term is below
-// f32 rounding).  Workgroup: 64 output rows x 64 outputs, 4 waves of 16 rows;
-// K steps of 32.  d_enc % 32 == 0.  Output rows are the frames of all
-// utterances packed in order (utterance u owns rows dst_row[u] ..
-// dst_row[u] + T[u]), so short windows of many utterances share tiles; a
-// row's utterance is the last u with dst_row[u] <= row.
-constexpr int kEpTile = 64, kEpK = 32, kEpStride = kEpK + 8;   // LDS row stride in halves
-// The global loads of K step k+1 are issued before the products of step k (one
-// register set ahead), so each step waits for LDS and the matrix cores rather
-// than for memory.  Threads of the whole grid also zero `clear_words` 32-bit
+// GEMM with f32 accuracy.  Frames (f32) are split into f16 hi + lo.  How W_e
+// arrives, by its storage (kEp*):
+//   quantised  the block integers as exact f16 [J][D] and the block scales as
+//              f32 [D/32][J]: per K block p = q.lo(q.hi), acc += scale * p;
+//   f16        as stored [J][D]: acc += w.hi, then w.lo;
+//   f32        hi and lo planes [J][D]: acc += hi.hi, hi.lo (frames' lo), lo.hi
+//              (the lo.lo term is below f32 rounding).
+// K blocks of 32 in order, one accumulator per output: the three kernels below
+// run the same instructions per output, so their rows are equal bit for bit and
+// the host chooses between them by row count alone.
+// Against hi and lo planes of the dequantised weights for every storage type, a K
+// block takes 2 MFMAs instead of 3 and its error against 64 bits falls (joint
+// logits of TDT-0.6b q8_0: 3.0e-7 against 4.1e-7 relative): the integers are exact,
+// while the lo plane of a small weight is a subnormal f16.
+// d_enc % 32 == 0.  Output rows are the frames of all utterances packed in order
+// (utterance u owns rows dst_row[u] .. dst_row[u] + T[u]), so short windows of
+// many utterances share tiles; a row's utterance is the last u with
+// dst_row[u] <= row.  Threads of the whole grid also zero `clear_words` 32-bit
 // words at `clear` (the decode loop's status, barrier flags and argmax keys),
 // which saves the loop a separate fill.
-__global__ void __launch_bounds__(256) enc_proj_kernel(const _Float16 *__restrict whi, const _Float16 *__restrict wlo,
-                                                       int J, const float *__restrict bias,
-                                                       const float *__restrict enc, int d_enc,
-                                                       const long long *__restrict src_row,
-                                                       const long long *__restrict dst_row, int n_utts,
-                                                       long long rows, float *__restrict out,
-                                                       unsigned *__restrict clear, size_t clear_words) {
-    __shared__ __attribute__((aligned(16))) _Float16 ah[kEpTile * kEpStride], al[kEpTile * kEpStride];
-    __shared__ __attribute__((aligned(16))) _Float16 bh[kEpTile * kEpStride], bl[kEpTile * kEpStride];
-    {
-        const size_t nthreads = (size_t)gridDim.x * gridDim.z * 256;
-        const size_t gtid = ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
-        for (size_t i = gtid; i < clear_words; i += nthreads) clear[i] = 0u;
+enum { kEpQuant = 0, kEpHalf = 1, kEpFull = 2 };
+struct EncProj {
+    const _Float16 *w, *w_lo;       // see above (w_lo: f32 only)
+    const float *w_scale;           // quantised only
+    const float *bias, *enc;
+    int J, d_enc, n_utts;
+    const long long *src_row, *dst_row;
+    long long rows;
+    float *out;
+    unsigned *clear;
+    size_t clear_words;
+};
+constexpr int kEpK = 32, kEpStride = kEpK + 8;   // K step; LDS row stride in halves
+
+__device__ __forceinline__ void ep_clear(const EncProj &e, size_t thread, size_t threads) {
+    for (size_t i = thread; i < e.clear_words; i += threads) e.clear[i] = 0u;
+}
+// First value of output row r's frame (rows past the last: the last row, never stored).
+__device__ __forceinline__ const float *ep_src(const EncProj &e, long long r) {
+    r = r < e.rows ? r : e.rows - 1;
+    int lo = 0, hi = e.n_utts - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (e.dst_row[mid] <= r) lo = mid;
+        else hi = mid - 1;
     }
+    return e.enc + (size_t)(e.src_row[lo] + (r - e.dst_row[lo])) * e.d_enc;
+}
+__device__ __forceinline__ void ep_split(const float4 &a, const float4 &b, half8 &h, half8 &l) {
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        h[i] = (_Float16)v[i];
+        l[i] = (_Float16)(v[i] - (float)h[i]);
+    }
+}
+// One K block of a 16x16 output tile (scale: kEpQuant, the lane's column).
+template <int W>
+__device__ __forceinline__ f32x4 ep_mma(half8 a_h, half8 a_l, half8 b, half8 b_lo, float scale, f32x4 acc) {
+    if constexpr (W == kEpQuant) {
+        f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_h, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        p = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_l, b, p, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = fmaf(scale, p[i], acc[i]);
+    } else {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_h, b, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_l, b, acc, 0, 0, 0);
+        if constexpr (W == kEpFull) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_h, b_lo, acc, 0, 0, 0);
+    }
+    return acc;
+}
+// D fragment of a tile: a lane holds output column `col` of rows row .. row + 3.
+__device__ __forceinline__ void ep_store(const EncProj &e, long long row, int col, f32x4 acc) {
+    if (col >= e.J) return;
+    const float bc = e.bias[col];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (row + i < e.rows) e.out[(size_t)(row + i) * e.J + col] = acc[i] + bc;
+}
+
+// Middle row counts: workgroup of 64 output rows x 64 outputs, 4 waves of 16
+// rows, K steps of 32 through LDS.  The global loads of K step k+1 are issued
+// before the products of step k (one register set ahead), so each step waits
+// for LDS and the matrix cores rather than for memory.
+constexpr int kEpTile = 64;
+template <int W>
+__global__ void __launch_bounds__(256) enc_proj_kernel(EncProj e) {
+    __shared__ __attribute__((aligned(16))) _Float16 ah[kEpTile * kEpStride], al[kEpTile * kEpStride];
+    __shared__ __attribute__((aligned(16))) _Float16 bh[kEpTile * kEpStride],
+        bl[W == kEpFull ? kEpTile * kEpStride : 8];
+    __shared__ float bs[W == kEpQuant ? kEpTile : 1];
+    ep_clear(e, ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * 256 + threadIdx.x, (size_t)gridDim.x * gridDim.z * 256);
     const long long m0 = (long long)blockIdx.x * kEpTile;
     const int n0 = blockIdx.z * kEpTile;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int sr = tid / 4, sc = (tid % 4) * 8;   // staging: row / column of this thread's 8 values
-    // the source frame of this thread's staging row
-    const long long r = m0 + sr;
-    const bool live = r < rows;
-    const float *src = enc;
-    if (live) {
-        int lo = 0, hi = n_utts - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (dst_row[mid] <= r) lo = mid;
-            else hi = mid - 1;
-        }
-        src = enc + (size_t)(src_row[lo] + (r - dst_row[lo])) * d_enc;
-    }
-    const int j = n0 + sr;
-    // one K step's global operands of this thread: 8 frame values, 8 W_e values (hi, lo)
-    float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f), v1 = v0;
-    half8 wh = half8{}, wl = half8{};
+    const float *src = ep_src(e, m0 + sr) + sc;
+    const size_t wrow = (size_t)min(n0 + sr, e.J - 1) * e.d_enc + sc;
+    const int scol = min(n0 + tid, e.J - 1);
+    // one K step's global operands of this thread
+    float4 v0, v1;
+    half8 wh, wl;
+    float ws = 0.f;
     auto fetch = [&](int k0) {
-        if (live) {
-            v0 = *reinterpret_cast<const float4 *>(src + k0 + sc);
-            v1 = *reinterpret_cast<const float4 *>(src + k0 + sc + 4);
-        }
-        if (j < J) {
-            wh = *reinterpret_cast<const half8 *>(whi + (size_t)j * d_enc + k0 + sc);
-            wl = *reinterpret_cast<const half8 *>(wlo + (size_t)j * d_enc + k0 + sc);
-        }
+        v0 = *reinterpret_cast<const float4 *>(src + k0);
+        v1 = *reinterpret_cast<const float4 *>(src + k0 + 4);
+        wh = *reinterpret_cast<const half8 *>(e.w + wrow + k0);
+        if constexpr (W == kEpFull) wl = *reinterpret_cast<const half8 *>(e.w_lo + wrow + k0);
+        if constexpr (W == kEpQuant)
+            if (tid < kEpTile) ws = e.w_scale[(size_t)(k0 / kEpK) * e.J + scol];
     };
     f32x4 acc[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     fetch(0);
-    for (int k0 = 0; k0 < d_enc; k0 += kEpK) {
+    for (int k0 = 0; k0 < e.d_enc; k0 += kEpK) {
         {
-            const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
             half8 h, l;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                h[i] = (_Float16)v[i];
-                l[i] = (_Float16)(v[i] - (float)h[i]);
-            }
+            ep_split(v0, v1, h, l);
             *reinterpret_cast<half8 *>(ah + sr * kEpStride + sc) = h;
             *reinterpret_cast<half8 *>(al + sr * kEpStride + sc) = l;
             *reinterpret_cast<half8 *>(bh + sr * kEpStride + sc) = wh;
-            *reinterpret_cast<half8 *>(bl + sr * kEpStride + sc) = wl;
+            if constexpr (W == kEpFull) *reinterpret_cast<half8 *>(bl + sr * kEpStride + sc) = wl;
+            if constexpr (W == kEpQuant)
+                if (tid < kEpTile) bs[tid] = ws;
         }
         __syncthreads();
-        if (k0 + kEpK < d_enc) fetch(k0 + kEpK);   // in flight during this step's products
+        if (k0 + kEpK < e.d_enc) fetch(k0 + kEpK);   // in flight during this step's products
         const int ao = (wave * 16 + (lane & 15)) * kEpStride + (lane >> 4) * 8;
         const half8 a_h = *reinterpret_cast<const half8 *>(ah + ao);
         const half8 a_l = *reinterpret_cast<const half8 *>(al + ao);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const int bo = (t * 16 + (lane & 15)) * kEpStride + (lane >> 4) * 8;
-            const half8 b_h = *reinterpret_cast<const half8 *>(bh + bo);
-            const half8 b_l = *reinterpret_cast<const half8 *>(bl + bo);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_h, b_h, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_l, b_h, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_h, b_l, acc[t], 0, 0, 0);
+            const half8 b = *reinterpret_cast<const half8 *>(bh + bo);
+            half8 b_lo = half8{};
+            if constexpr (W == kEpFull) b_lo = *reinterpret_cast<const half8 *>(bl + bo);
+            acc[t] = ep_mma<W>(a_h, a_l, b, b_lo, W == kEpQuant ? bs[t * 16 + (lane & 15)] : 0.f, acc[t]);
         }
         __syncthreads();
     }
-    // D fragment: lane holds output column 16t + lane % 16 of rows 4 (lane / 16) .. +3
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const int col = n0 + t * 16 + (lane & 15);
-        if (col >= J) continue;
-        const float bc = bias[col];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const long long row = m0 + wave * 16 + (lane >> 4) * 4 + i;
-            if (row < rows) out[(size_t)row * J + col] = acc[t][i] + bc;
-        }
-    }
+    for (int t = 0; t < 4; ++t)
+        ep_store(e, m0 + wave * 16 + (lane >> 4) * 4, n0 + t * 16 + (lane & 15), acc[t]);
 }
 
-// enc_proj for few rows (streaming chunks, short windows).  There the tiled
-// kernel above runs on a few dozen workgroups, each paying two workgroup
-// barriers and an LDS round trip per K step.  Here each wave owns one 16x16
-// output block and loads its operands straight into MFMA fragment registers,
-// kEnSteps K steps per batch, the next batch in flight while the current one is
-// multiplied: no LDS and no barrier.  Each block takes exactly the
-// instructions of enc_proj_kernel, in the same order: per K step of 32 the same
-// lane layout (row lane % 16, K slice 8 (lane / 16)), the same f16 hi / lo split
-// of the frames, hi.hi + lo.hi + hi.lo into one accumulator in K order, then +
-// bias.  So the two kernels' outputs are bit-identical, and the host chooses
-// between them by row count alone.  Workgroup: 4 waves, 16 rows x 64 outputs.
-constexpr int kEnSteps = 4;   // K steps per batch of the narrow kernel
-__global__ void __launch_bounds__(256) enc_proj_narrow_kernel(const _Float16 *__restrict whi,
-                                                              const _Float16 *__restrict wlo, int J,
-                                                              const float *__restrict bias,
-                                                              const float *__restrict enc, int d_enc,
-                                                              const long long *__restrict src_row,
-                                                              const long long *__restrict dst_row, int n_utts,
-                                                              long long rows, float *__restrict out,
-                                                              unsigned *__restrict clear, size_t clear_words) {
-    {
-        const size_t nthreads = (size_t)gridDim.x * gridDim.z * 256;
-        const size_t gtid = ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
-        for (size_t i = gtid; i < clear_words; i += nthreads) clear[i] = 0u;
+// Large row counts (batched offline decoding): workgroup of 128 output rows x
+// 320 outputs, 8 waves of 64 x 80 (4 x 5 tiles).  A frame is split and staged
+// J / 320 times instead of J / 64 times and read from LDS by 4 waves instead of
+// one per 4 tiles; per K step a wave reads 13 KB of fragments from LDS for 40
+// MFMAs (64 x 64 tiles: 6 KB for 12).  Two LDS buffers, one barrier per K step:
+// step k+1 is written from registers and step k+2's loads are issued before the
+// products of step k (loads one more step ahead measured the same).  Workgroups
+// that share rows sit on one XCD (ids 8 apart), one after the other, so the second
+// reads the frames from its L2.
+// 131,072 rows, D = 1024, J = 640: q8_0 481 us, f16 446 us, f32 605 us (0.71, 0.77,
+// 0.85 PFLOP/s of MFMA; a large library product reaches 1.21 on the same card), 1279,
+// 1285 and 1408 us with enc_proj_kernel.  It is bound by the workgroup's serial K
+// steps, about 1.5 us each, so a launch takes 50 us however few its rows are: up to
+// 8,192 rows the 64 x 64 tiles are as fast or faster (51 against 55 us; 16,384 rows:
+// 94 against 59), hence the host's line (kWideRows) between the two.
+constexpr int kEwRows = 128, kEwCols = 320, kEwThreads = 512;
+template <int W>
+__global__ void __launch_bounds__(kEwThreads) enc_proj_wide_kernel(EncProj e) {
+    __shared__ __attribute__((aligned(16))) _Float16 ah[2][kEwRows * kEpStride], al[2][kEwRows * kEpStride];
+    __shared__ __attribute__((aligned(16))) _Float16 bh[2][kEwCols * kEpStride],
+        bl[2][W == kEpFull ? kEwCols * kEpStride : 8];
+    __shared__ float bs[2][W == kEpQuant ? kEwCols : 1];
+    ep_clear(e, (size_t)blockIdx.x * kEwThreads + threadIdx.x, (size_t)gridDim.x * kEwThreads);
+    const int n_col = (e.J + kEwCols - 1) / kEwCols, group = blockIdx.x / (8 * n_col), in = blockIdx.x % (8 * n_col);
+    const long long m0 = (long long)(group * 8 + (in & 7)) * kEwRows;
+    const int n0 = (in >> 3) * kEwCols;
+    if (m0 >= e.rows) return;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int wr = (wave >> 2) * 64, wn = (wave & 3) * 80;   // this wave's rows and columns of the tile
+    const int sr = tid / 4, sc = (tid % 4) * 8;              // staging: one row's 8 values, 3 columns' 8 values
+    const float *src = ep_src(e, m0 + sr) + sc;
+    constexpr int kChunks = kEwCols * 4, kPer = (kChunks + kEwThreads - 1) / kEwThreads;
+    size_t wrow[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) wrow[i] = (size_t)min(n0 + (tid + i * kEwThreads) / 4, e.J - 1) * e.d_enc + sc;
+    const int scol = min(n0 + tid, e.J - 1);
+    float4 v0, v1;
+    half8 wh[kPer], wl[kPer];
+    float ws = 0.f;
+    auto fetch = [&](int k0) {
+        v0 = *reinterpret_cast<const float4 *>(src + k0);
+        v1 = *reinterpret_cast<const float4 *>(src + k0 + 4);
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            wh[i] = *reinterpret_cast<const half8 *>(e.w + wrow[i] + k0);
+            if constexpr (W == kEpFull) wl[i] = *reinterpret_cast<const half8 *>(e.w_lo + wrow[i] + k0);
+        }
+        if constexpr (W == kEpQuant) ws = e.w_scale[(size_t)(k0 / kEpK) * e.J + scol];
+    };
+    auto stage = [&](int b) {
+        half8 h, l;
+        ep_split(v0, v1, h, l);
+        *reinterpret_cast<half8 *>(ah[b] + sr * kEpStride + sc) = h;
+        *reinterpret_cast<half8 *>(al[b] + sr * kEpStride + sc) = l;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int col = (tid + i * kEwThreads) / 4;
+            if ((i + 1) * kEwThreads > kChunks && col >= kEwCols) break;
+            *reinterpret_cast<half8 *>(bh[b] + col * kEpStride + sc) = wh[i];
+            if constexpr (W == kEpFull) *reinterpret_cast<half8 *>(bl[b] + col * kEpStride + sc) = wl[i];
+        }
+        if constexpr (W == kEpQuant)
+            if (tid < kEwCols) bs[b][tid] = ws;
+    };
+    f32x4 acc[4][5];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int n = 0; n < 5; ++n) acc[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int steps = e.d_enc / kEpK, last = e.d_enc - kEpK;
+    fetch(0);
+    stage(0);
+    fetch(min(kEpK, last));   // (steps past the last reload it)
+    lds_sync();
+    const int fo = (lane & 15) * kEpStride + (lane >> 4) * 8;
+    for (int s = 0; s < steps; ++s) {
+        const int b = s & 1;
+        // the other buffer's readers, step s-1, are behind the last barrier
+        if (s + 1 < steps) stage(b ^ 1);
+        fetch(min((s + 2) * kEpK, last));
+        half8 a_h[4], a_l[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            a_h[t] = *reinterpret_cast<const half8 *>(ah[b] + (wr + t * 16) * kEpStride + fo);
+            a_l[t] = *reinterpret_cast<const half8 *>(al[b] + (wr + t * 16) * kEpStride + fo);
+        }
+#pragma unroll
+        for (int n = 0; n < 5; ++n) {
+            const int bo = (wn + n * 16) * kEpStride + fo;
+            const half8 w = *reinterpret_cast<const half8 *>(bh[b] + bo);
+            half8 w_lo = half8{};
+            if constexpr (W == kEpFull) w_lo = *reinterpret_cast<const half8 *>(bl[b] + bo);
+            const float scale = W == kEpQuant ? bs[b][wn + n * 16 + (lane & 15)] : 0.f;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t][n] = ep_mma<W>(a_h[t], a_l[t], w, w_lo, scale, acc[t][n]);
+        }
+        lds_sync();
     }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int n = 0; n < 5; ++n)
+            ep_store(e, m0 + wr + t * 16 + (lane >> 4) * 4, n0 + wn + n * 16 + (lane & 15), acc[t][n]);
+}
+
+// Few rows (streaming chunks, short windows).  There the tiled kernels above run
+// on a few dozen workgroups, each paying workgroup barriers and an LDS round trip
+// per K step.  Here each wave owns one 16x16 output block and loads its operands
+// straight into MFMA fragment registers, kEnSteps K steps per batch, the next
+// batch in flight while the current one is multiplied: no LDS and no barrier.
+// Workgroup: 4 waves, 16 rows x 64 outputs.
+constexpr int kEnSteps = 4;   // K steps per batch of the narrow kernel
+template <int W>
+__global__ void __launch_bounds__(256) enc_proj_narrow_kernel(EncProj e) {
+    ep_clear(e, ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * 256 + threadIdx.x, (size_t)gridDim.x * gridDim.z * 256);
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const long long m0 = (long long)blockIdx.x * 16;
     const int n0 = (blockIdx.z * 4 + wave) * 16;
-    if (n0 >= J) return;
-    const long long r = m0 + (lane & 15);
-    const bool live = r < rows;
-    const float *src = enc;
-    if (live) {
-        int lo = 0, hi = n_utts - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (dst_row[mid] <= r) lo = mid;
-            else hi = mid - 1;
-        }
-        src = enc + (size_t)(src_row[lo] + (r - dst_row[lo])) * d_enc;
-    }
-    const int col = n0 + (lane & 15);
-    const bool cl = col < J;
+    if (n0 >= e.J) return;
+    const int col = n0 + (lane & 15), cc = min(col, e.J - 1);
     const int ks = (lane >> 4) * 8;
-    const int nsteps = d_enc / kEpK, nb = (nsteps + kEnSteps - 1) / kEnSteps;
-    // Every lane loads: a row past the last reads frame row 0 and a column past J reads
-    // W_e row J - 1.  Row i of an MFMA product depends only on row i of A, and column j
+    const int nsteps = e.d_enc / kEpK, nb = (nsteps + kEnSteps - 1) / kEnSteps;
+    // Every lane loads: a row past the last reads the last frame row and a column past J
+    // reads W_e row J - 1.  Row i of an MFMA product depends only on row i of A, and column j
     // only on column j of B, so those lanes' values reach only outputs never stored.
-    const _Float16 *bhp = whi + (size_t)(cl ? col : J - 1) * d_enc + ks;
-    const _Float16 *blp = wlo + (size_t)(cl ? col : J - 1) * d_enc + ks;
-    src += ks;
+    const float *src = ep_src(e, m0 + (lane & 15)) + ks;
+    const _Float16 *bhp = e.w + (size_t)cc * e.d_enc + ks;
+    const _Float16 *blp = W == kEpFull ? e.w_lo + (size_t)cc * e.d_enc + ks : nullptr;
     struct Batch {
         float4 a0[kEnSteps], a1[kEnSteps];
         half8 bh[kEnSteps], bl[kEnSteps];
+        float s[kEnSteps];
     };
     // batch b's operands (a batch past the last reloads the last one, so no load sits
     // behind a branch and the compiler's wait counts stay exact)
@@ -514,7 +631,9 @@ __global__ void __launch_bounds__(256) enc_proj_narrow_kernel(const _Float16 *__
             x.a0[s] = *reinterpret_cast<const float4 *>(src + k);
             x.a1[s] = *reinterpret_cast<const float4 *>(src + k + 4);
             x.bh[s] = *reinterpret_cast<const half8 *>(bhp + k);
-            x.bl[s] = *reinterpret_cast<const half8 *>(blp + k);
+            x.bl[s] = half8{};
+            if constexpr (W == kEpFull) x.bl[s] = *reinterpret_cast<const half8 *>(blp + k);
+            x.s[s] = W == kEpQuant ? e.w_scale[(size_t)st * e.J + cc] : 0.f;
         }
     };
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -522,17 +641,9 @@ __global__ void __launch_bounds__(256) enc_proj_narrow_kernel(const _Float16 *__
 #pragma unroll
         for (int s = 0; s < kEnSteps; ++s) {
             if (b * kEnSteps + s >= nsteps) break;
-            const float v[8] = {x.a0[s].x, x.a0[s].y, x.a0[s].z, x.a0[s].w,
-                                x.a1[s].x, x.a1[s].y, x.a1[s].z, x.a1[s].w};
             half8 h, l;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                h[i] = (_Float16)v[i];
-                l[i] = (_Float16)(v[i] - (float)h[i]);
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(h, x.bh[s], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(l, x.bh[s], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(h, x.bl[s], acc, 0, 0, 0);
+            ep_split(x.a0[s], x.a1[s], h, l);
+            acc = ep_mma<W>(h, l, x.bh[s], x.bl[s], x.s[s], acc);
         }
     };
     Batch X, Y;
@@ -543,13 +654,7 @@ __global__ void __launch_bounds__(256) enc_proj_narrow_kernel(const _Float16 *__
         load(b + 2, X);
         if (b + 1 < nb) mul(b + 1, Y);
     }
-    if (!cl) return;
-    const float bc = bias[col];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const long long row = m0 + (lane >> 4) * 4 + i;
-        if (row < rows) out[(size_t)row * J + col] = acc[i] + bc;
-    }
+    ep_store(e, m0 + (lane >> 4) * 4, col, acc);
 }
 
 // ---------------------------------------------------------------- decode loop
