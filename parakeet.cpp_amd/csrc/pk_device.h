@@ -245,6 +245,34 @@ __device__ __forceinline__ f32x4 quad_transpose(f32x4 a) {
     return a;
 }
 
+// Maximum of a 64-bit value over the lanes that agree modulo `step` (a power of two up to 16),
+// in every lane.  Below 16 by rotations inside a DPP row of 16 lanes, then by the row and half
+// swaps: no LDS round trip (a shuffle is one, about 0.05 us, and an argmax takes up to six).
+typedef unsigned long long u64;
+template <int CTRL>
+__device__ __forceinline__ u64 row_ror_max(u64 v) {
+    const unsigned lo = __builtin_amdgcn_mov_dpp((int)(unsigned)v, CTRL, 0xF, 0xF, false);
+    const unsigned hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(v >> 32), CTRL, 0xF, 0xF, false);
+    const u64 o = ((u64)hi << 32) | lo;
+    return o > v ? o : v;
+}
+__device__ __forceinline__ u64 lanes_max(u64 v, int step) {
+    if (step <= 8) v = row_ror_max<0x128>(v);   // row_ror:8
+    if (step <= 4) v = row_ror_max<0x124>(v);
+    if (step <= 2) v = row_ror_max<0x122>(v);
+    if (step <= 1) v = row_ror_max<0x121>(v);
+    if (step <= 16) {   // rows 0, 1 and rows 2, 3
+        const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
+        const u64 a = ((u64)hi[0] << 32) | lo[0], b = ((u64)hi[1] << 32) | lo[1];
+        v = a > b ? a : b;
+    }
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
+    const u64 a = ((u64)hi[0] << 32) | lo[0], b = ((u64)hi[1] << 32) | lo[1];
+    return a > b ? a : b;
+}
+
 // Staged activation block: 16 utterance rows of K values as f16 (hi, lo).
 // Only rows 0 .. n-1 are staged; product columns n .. 15 are not used.
 struct Act {
@@ -271,8 +299,8 @@ __device__ __forceinline__ unsigned ordered_bits(float v) {
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 // Larger key = larger value, then smaller index: the reference's first-index rule.
-__device__ __forceinline__ unsigned long long make_key(float v, int idx) {
-    return ((unsigned long long)ordered_bits(v) << kIdxBits) | (unsigned long long)((1 << kIdxBits) - 1 - idx);
+__device__ __forceinline__ unsigned long long make_key(unsigned ordered, int idx) {
+    return ((unsigned long long)ordered << kIdxBits) | (unsigned long long)((1 << kIdxBits) - 1 - idx);
 }
 __device__ __forceinline__ int key_index(unsigned long long key) {
     return (1 << kIdxBits) - 1 - (int)(key & ((1u << kIdxBits) - 1));
@@ -659,26 +687,41 @@ __global__ void __launch_bounds__(256) enc_proj_narrow_kernel(EncProj e) {
 
 // ---------------------------------------------------------------- decode loop
 
-struct Ctl {                      // per-workgroup copy of its domain's control state
-    int b[kDomCap];               // batch index of each domain utterance
-    int t[kDomCap], T[kDomCap], sym[kDomCap], pend[kDomCap], flags[kDomCap];
-    int ntok[kDomCap], steps[kDomCap], nseg[kDomCap], segst[kDomCap], last[kDomCap];
-    int cur[kDomCap];             // parity of the utterance's state once its pending token (if any) is taken
-    int lst[kDomCap], jst[kDomCap];
-    int stp[kDomCap];             // 1: the utterance took an LSTM step in this launch
-    // joint columns: column i < nj is joint-list utterance i at its frame t; columns
-    // sbase[i] .. sbase[i] + sn[i] - 1 are the same utterance at frames t + 1 .. t + sn[i]
-    int cu[kColCap], co[kColCap], sbase[kDomCap], sn[kDomCap];
-    long long crow[kColCap];      // encp row of each column (utterance's first row + t + offset)
-    int cb[kColCap];              // batch index of each column's utterance
-    int brun[kDomCap];            // 1: the utterance's last decision kept the prediction output
-    int ncol;
-    long long erow[kDomCap];      // first encp row of each utterance
-    float bbias[kDomCap];         // blank logit offset of each utterance
+// Control state of an utterance of the domain: lane ul of wave 0 holds utterance ul's for
+// the whole launch, in registers (the other waves' copies are not used).  The decisions
+// are a serial chain in which every workgroup waits; with this state in LDS every field
+// was a dependent round trip of 0.05 us.  The lists go out as the byte offsets their
+// readers need (Ctl::lrow, crow), one LDS read instead of list entry, fields and products.
+// Measured with the joint's epilogue on ordered bits (joint_phase), us per iteration before
+// and after: B=1 13.61 -> 12.57, B=24 (TDT-1.1b f16) 18.29 -> 17.11, EOU-120m B=16 13.06 ->
+// 11.93, B=64 19.83 -> 19.39, B=256 32.12 -> 31.22, B=512 41.69 -> 39.57.
+struct Utt {
+    int t, T, sym, pend, flags, ntok, steps;
+    int cur;                      // parity of the utterance's state once its pending token (if any) is taken
+    int keep;                     // 1: the last decision kept the prediction output
+    int stp;                      // 1: the utterance took an LSTM step in this launch
+    // joint columns: column col is the utterance at its frame t; columns sbase .. sbase + sn - 1
+    // are the same utterance at frames t + 1 .. t + sn
+    int col, sbase, sn;
+};
+
+struct Ctl {                      // per-workgroup state of its domain
+    // the lists of an iteration, as the byte offsets their readers need
+    int4 cnt;                     // LSTM list length, joint list length, joint columns, log2 of the first, rounded up
+    // LSTM list row: E' row of the pending token; c_0 row of the old state (-1: zero state) and of the
+    // new one; h row | parity << 6 | zero state << 5 | domain utterance
+    int4 lrow[kDomCap];
+    int4 crow[kColCap];           // joint column: encp row, ppx row, blank offset (f32 bits), -
+    // per domain utterance, for the whole launch
+    int b[kDomCap];               // batch index
+    unsigned erow[kDomCap];       // first encp row (byte offset)
+    float bbias[kDomCap];         // blank logit offset
     int tbase[kDomCap];           // tokens before this call (EOU segment indices)
+    int nseg[kDomCap], segst[kDomCap], last[kDomCap];   // EOU (lane ul of wave 0)
+    int cur[kDomCap];             // parity of the state at the start and at the end
+    int mark[kDomCap];            // start: 1 = zero state; end: 1 = took an LSTM step
     int dur[PK_MAX_DURATIONS];    // duration values (the decision step reads them from LDS)
-    int n, nl, nj;
-    int lgn;                      // log2 of the LSTM list length, rounded up
+    int n;
     int dom, rank, P;
     int ok;                       // 0: a wait ended without its data (error or time-out)
     // this workgroup's tiles of an LSTM matrix, of W_p and of W_o (fixed for the
@@ -692,6 +735,8 @@ struct Ctl {                      // per-workgroup copy of its domain's control 
     unsigned long long wgkey[kColCap][2];   // this workgroup's best key per joint column and head
     unsigned long long prof[kPrN];
 };
+// Row word of the LSTM list (rows of h are multiples of 128 bytes).
+constexpr int kRowUl = 31, kRowZero = 32, kRowCur = 64, kRowMask = ~127;
 
 __device__ __forceinline__ void pmark(const KParams &p, Ctl &s, unsigned long long &last, int k) {
     if (!p.prof) return;
@@ -725,6 +770,22 @@ __device__ __forceinline__ unsigned long long *tl_t0() { __shared__ unsigned lon
 #define TL(k) TLX(k, 1)
 #define TLA(k) TLX(k, 0)
 
+// State offsets (floats): c_0 / h_0 of parity buf, W_hh0 . h_0.
+__device__ __forceinline__ size_t cx_off(const KParams &p, int buf, int b) { return ((size_t)buf * p.n_utts + b) * p.H; }
+__device__ __forceinline__ size_t rx_off(const KParams &p, int buf, int b) {
+    return ((size_t)buf * p.n_utts + b) * 4 * p.H;
+}
+__device__ __forceinline__ size_t hs_off(const KParams &p, int layer, int b) {
+    return ((size_t)layer * p.n_utts + b) * p.H;
+}
+// Exchange offsets (floats): the 4 units of tile t for list row u; the 16 rows
+// of pred tile t for domain utterance ul.
+__device__ __forceinline__ unsigned hx_at(const KParams &p, int dom, int layer, int half, int t, int u) {
+    return ((((unsigned)((layer - p.hl0) * 2 + half) * p.n_dom + dom) * (p.H / 4) + t) * p.rows + u) * 4u;
+}
+__device__ __forceinline__ unsigned ppx_at(const KParams &p, int dom, int half, int t, int ul) {
+    return ((((unsigned)half * p.n_dom + dom) * (p.J / kTile) + t) * p.prows + ul) * (unsigned)kTile;
+}
 // Compact the LSTM list (pending token) and the joint list (frames left).
 // Then the joint columns: one per joint-list utterance at its frame t, and
 // (spec) the column tiles' spare columns dealt out evenly as frames t + 1,
@@ -733,35 +794,40 @@ __device__ __forceinline__ unsigned long long *tl_t0() { __shared__ unsigned lon
 // prediction output, so the logits of the next frame are already in a spare
 // column: the decision step walks a run of blanks in one iteration instead of
 // one iteration per blank.
-__device__ __forceinline__ void build_lists(Ctl &s, bool spec) {
+__device__ __forceinline__ void build_lists(const KParams &p, Ctl &s, Utt &u) {
     if (threadIdx.x < kWave) {
-        const int lane = threadIdx.x;
-        const bool fl = lane < s.n && s.pend[lane] >= 0;
-        const bool fj = lane < s.n && s.t[lane] < s.T[lane];
+        const int lane = threadIdx.x, ul = min(lane, kDomCap - 1);
+        const bool fl = lane < s.n && u.pend >= 0;
+        const bool fj = lane < s.n && u.t < u.T;
         const unsigned long long bl = __ballot(fl), bj = __ballot(fj);
         const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
         const int il = __popcll(bl & below), ij = __popcll(bj & below);
-        if (fl) s.lst[il] = lane;
-        if (fj) s.jst[ij] = lane;
+        const int b = s.b[ul];
+        if (fl) {
+            const bool zero = u.flags & kFlagZeroHC;
+            const int row = p.H * 4;   // bytes of a c_0 row
+            s.lrow[il] = make_int4(u.pend * 4 * row, zero ? -1 : ((u.cur ^ 1) * p.n_utts + b) * row,
+                                   (u.cur * p.n_utts + b) * row,
+                                   b * row | (u.cur ? kRowCur : 0) | (zero ? kRowZero : 0) | lane);
+        }
         const int nj = __popcll(bj);
         // an utterance in a blank run takes q spare columns: an even share of the
         // spare columns of the tiles, capped at the frames it has left
-        const int spare = spec && nj > 0 ? ((nj + kTile - 1) / kTile) * kTile - nj : 0;
-        const bool fe = fj && spare > 0 && s.brun[lane] != 0;
+        const int spare = p.spec != 0 && nj > 0 ? ((nj + kTile - 1) / kTile) * kTile - nj : 0;
+        const bool fe = fj && spare > 0 && u.keep != 0;
         const unsigned long long be = __ballot(fe);
         int total = 0;
-        if (fj) {
-            s.cu[ij] = lane;
-            s.co[ij] = 0;
-            s.crow[ij] = s.erow[lane] + s.t[lane];
-            s.cb[ij] = s.b[lane];
-        }
+        int4 c = make_int4((int)(s.erow[ul] + (unsigned)u.t * (unsigned)(p.J * 4)),
+                           (int)(ppx_at(p, s.dom, u.cur, 0, ul) * 4u), __float_as_int(s.bbias[ul]), 0);
+        if (fj) s.crow[ij] = c;
+        u.col = ij;
+        u.sbase = u.sn = 0;
         if (be != 0ull) {   // some utterance is in a run of blanks (wave-uniform)
             const int ne = __popcll(be), ie = __popcll(be & below);
             int q = 0;
             if (fe) {
                 q = spare / ne + (ie < spare % ne ? 1 : 0);
-                q = min(q, s.T[lane] - s.t[lane] - 1);
+                q = min(q, u.T - u.t - 1);
             }
             // exclusive prefix sum of q over the joint list (lanes in list order)
             int incl = q;
@@ -771,24 +837,18 @@ __device__ __forceinline__ void build_lists(Ctl &s, bool spec) {
                 if (lane >= d) incl += v;
             }
             if (fj) {
-                const int base = nj + incl - q;
-                s.sbase[ij] = base;
-                s.sn[ij] = q;
+                u.sbase = nj + incl - q;
+                u.sn = q;
                 for (int o = 1; o <= q; ++o) {
-                    s.cu[base + o - 1] = lane;
-                    s.co[base + o - 1] = o;
-                    s.crow[base + o - 1] = s.erow[lane] + s.t[lane] + o;
-                    s.cb[base + o - 1] = s.b[lane];
+                    c.x += p.J * 4;
+                    s.crow[u.sbase + o - 1] = c;
                 }
             }
             total = __shfl(incl, kWave - 1, kWave);
         }
         if (lane == 0) {
             const int nl = __popcll(bl);
-            s.nl = nl;
-            s.lgn = nl <= 1 ? 0 : 32 - __builtin_clz((unsigned)(nl - 1));
-            s.nj = nj;
-            s.ncol = nj + total;
+            s.cnt = make_int4(nl, nj, nj + total, nl <= 1 ? 0 : 32 - __builtin_clz((unsigned)(nl - 1)));
         }
     }
     lds_sync();
@@ -859,22 +919,6 @@ __device__ __forceinline__ bool dom_sync(const KParams &p, Ctl &s, unsigned &epo
 // waits for all of its own stores before that, so a workgroup that has seen
 // every key sees every word emptied or written in the iteration.
 
-// State offsets (floats): c_0 / h_0 of parity buf, W_hh0 . h_0.
-__device__ __forceinline__ size_t cx_off(const KParams &p, int buf, int b) { return ((size_t)buf * p.n_utts + b) * p.H; }
-__device__ __forceinline__ size_t rx_off(const KParams &p, int buf, int b) {
-    return ((size_t)buf * p.n_utts + b) * 4 * p.H;
-}
-__device__ __forceinline__ size_t hs_off(const KParams &p, int layer, int b) {
-    return ((size_t)layer * p.n_utts + b) * p.H;
-}
-// Exchange offsets (floats): the 4 units of tile t for list row u; the 16 rows
-// of pred tile t for domain utterance ul.
-__device__ __forceinline__ unsigned hx_at(const KParams &p, int dom, int layer, int half, int t, int u) {
-    return ((((unsigned)((layer - p.hl0) * 2 + half) * p.n_dom + dom) * (p.H / 4) + t) * p.rows + u) * 4u;
-}
-__device__ __forceinline__ unsigned ppx_at(const KParams &p, int dom, int half, int t, int ul) {
-    return ((((unsigned)half * p.n_dom + dom) * (p.J / kTile) + t) * p.prows + ul) * (unsigned)kTile;
-}
 // A produced word: never the empty pattern (a NaN that loses one payload bit).
 __device__ __forceinline__ float filled(float v) {
     const unsigned b = __float_as_uint(v);
@@ -1403,10 +1447,10 @@ __device__ __forceinline__ void cache_matrix(const TMat &m, int rank, int P, uns
 // the iteration: the list rebuild has fixed every column's frame, and the loads
 // complete during layer 0, whose own loads take as long, instead of at the
 // joint's staging.
-__device__ __forceinline__ void encp_prefetch(const KParams &p, const Ctl &s, const Bufs &B, float4 (&e)[kStageMax]) {
+__device__ __forceinline__ void encp_prefetch(const KParams &p, const Ctl &s, const Bufs &B, int ncol, float4 (&e)[kStageMax]) {
     const int J = p.J, ntile = J / kTile, g = threadIdx.x & 3, u = (threadIdx.x >> 2) & 15, t0 = threadIdx.x >> 6;
-    const bool live = u < min(kTile, s.ncol);
-    const unsigned erow = (unsigned)((size_t)s.crow[live ? u : 0] * J * 4);
+    const bool live = u < min(kTile, ncol);
+    const unsigned erow = (unsigned)s.crow[live ? u : 0].x;
 #pragma unroll
     for (int j = 0; j < kStageMax; ++j) {
         const int t = t0 + kWaves * j;
@@ -1415,22 +1459,21 @@ __device__ __forceinline__ void encp_prefetch(const KParams &p, const Ctl &s, co
 }
 
 template <int WC>
-__device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs &B, const Lds &S, unsigned stamp,
+__device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs &B, const Lds &S, unsigned stamp, int ncol,
                             const float4 (&epre)[kStageMax], unsigned long long &tlast) {
     const int J = p.J, lane = threadIdx.x & (kWave - 1);
     if (threadIdx.x < 2 * kColCap) s.wgkey[threadIdx.x / 2][threadIdx.x % 2] = 0ull;
     const int n_out = s.own_out;
-    for (int c0 = 0; c0 < s.ncol; c0 += kTile) {
-        const int nc = min(kTile, s.ncol - c0);
+    for (int c0 = 0; c0 < ncol; c0 += kTile) {
+        const int nc = min(kTile, ncol - c0);
         Act x = S.act[0];
         x.n = nc;
         // stage hidden = relu(encp[t] + pp) for this column tile
         {
             const int ntile = J / kTile, g = threadIdx.x & 3, u = (threadIdx.x >> 2) & 15, t0 = threadIdx.x >> 6;
             const bool live = u < nc;
-            const int col = c0 + (live ? u : 0), ul = s.cu[col];
-            const unsigned erow = (unsigned)((size_t)s.crow[col] * J * 4);
-            const unsigned prow = (ppx_at(p, s.dom, s.cur[ul], 0, ul) + g * 4) * 4u;
+            const int2 row = *reinterpret_cast<const int2 *>(&s.crow[c0 + (live ? u : 0)]);
+            const unsigned erow = (unsigned)row.x, prow = (unsigned)row.y + g * 16u;
             const unsigned stride = (unsigned)p.prows * kTile * 4u;
             for (int b0 = 0; b0 < ntile; b0 += kWaves * kStageMax) {
                 float4 e[kStageMax];
@@ -1472,7 +1515,7 @@ __device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs
         // rows 4g .. 4g+3 of a tile for utterance u of the column tile; its blank
         // offset is loaded before the products
         const int u = 4 * (lane >> 4) + (lane & 3), g = (lane >> 2) & 3;
-        const float bb = u < nc ? s.bbias[s.cu[c0 + u]] : 0.0f;
+        const float bb = u < nc ? __int_as_float(s.crow[c0 + u].z) : 0.0f;
         // (b_out is zero-padded to whole tiles)
         const float *btab = S.bias + kTile * ((p.L - 1) * s.own_lstm + s.own_pred);
         TL(1);
@@ -1480,52 +1523,69 @@ __device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs
         // the decision step copies a column to the row of the step that takes it
         float *ltap = nullptr;
         if (p.logits && u < nc) ltap = p.lcol + ((size_t)s.dom * kColCap + c0 + u) * p.Vo;
-        // each lane keeps its best key per head over all its rows; the four
-        // lanes of one utterance then combine, and one LDS atomic per utterance
-        // and head follows
-        unsigned long long best0 = 0ull, best1 = 0ull;
+        // each lane keeps the best value (as ordered bits, never 0) and row of each head:
+        // its rows come in ascending order, so "greater" keeps the first index; the four
+        // lanes of one utterance then combine, and one LDS atomic per utterance and
+        // head follows.  (64-bit keys per row, with the head, the range and the blank
+        // tested row by row, made the reduce of a 24-tile pass 2.4 us; with one test per
+        // tile and 32-bit compares the joint's products and reduce fall from 11.0 to
+        // 10.2 us at B = 256 and from 17.1 to 15.9 at B = 512.)
+        unsigned top0 = 0u, top1 = 0u;
+        int row0 = 0, row1 = 0;
         run_phase<WC>(p.w_out, n_out, p.w_out, n_out, s.rank, s.P, x, S.red, S.wcache, s.pass[p.L],
                   [&](int k, f32x4 acc) {
                       acc = quad_transpose(acc);   // every lane of the wave takes part
-                      if (u >= nc) return;
-                      const int tile = s.rank + k * s.P;
+                      const int tile = s.rank + k * s.P, first = tile * kTile;   // wave-uniform
                       const float4 bias4 = *reinterpret_cast<const float4 *>(btab + k * kTile + g * 4);
+                      float v[4] = {acc[0] + bias4.x, acc[1] + bias4.y, acc[2] + bias4.z, acc[3] + bias4.w};
+                      if ((unsigned)(p.blank - first) < (unsigned)kTile) {
 #pragma unroll
-                      for (int i = 0; i < 4; ++i) {
-                          const int row = tile * kTile + g * 4 + i;
-                          if (row >= p.Vo) continue;
-                          const float bias = i == 0 ? bias4.x : i == 1 ? bias4.y : i == 2 ? bias4.z : bias4.w;
-                          float v = acc[i] + bias;
-                          if (row == p.blank) v += bb;
-                          if (ltap) st_coh(ltap + row, v);
-                          if (row < p.V1) {
-                              const unsigned long long key = make_key(v, row);
-                              best0 = key > best0 ? key : best0;
-                          } else {
-                              const unsigned long long key = make_key(v, row - p.V1);
-                              best1 = key > best1 ? key : best1;
+                          for (int i = 0; i < 4; ++i)
+                              if (first + g * 4 + i == p.blank) v[i] += bb;
+                      }
+                      if (ltap) {
+#pragma unroll
+                          for (int i = 0; i < 4; ++i)
+                              if (first + g * 4 + i < p.Vo) st_coh(ltap + first + g * 4 + i, v[i]);
+                      }
+                      if (first + kTile <= p.V1) {   // token rows only
+#pragma unroll
+                          for (int i = 0; i < 4; ++i) {
+                              const unsigned o = max(ordered_bits(v[i]), 1u);
+                              const bool better = o > top0;
+                              top0 = better ? o : top0;
+                              row0 = better ? first + g * 4 + i : row0;
+                          }
+                      } else {
+#pragma unroll
+                          for (int i = 0; i < 4; ++i) {
+                              const int row = first + g * 4 + i;
+                              const unsigned o = max(ordered_bits(v[i]), 1u);
+                              const bool b0 = row < p.V1 && o > top0, b1 = row >= p.V1 && row < p.Vo && o > top1;
+                              top0 = b0 ? o : top0;
+                              row0 = b0 ? row : row0;
+                              top1 = b1 ? o : top1;
+                              row1 = b1 ? row - p.V1 : row1;
                           }
                       }
                   });
-#pragma unroll
-        for (int m = 4; m < kTile; m <<= 1) {   // the lanes of utterance u differ in bits 2 and 3
-            const unsigned long long o0 = __shfl_xor(best0, m, kWave), o1 = __shfl_xor(best1, m, kWave);
-            best0 = o0 > best0 ? o0 : best0;
-            best1 = o1 > best1 ? o1 : best1;
-        }
+        // the lanes of utterance u differ in bits 2 and 3
+        u64 best0 = top0 != 0u ? make_key(top0, row0) : 0ull, best1 = top1 != 0u ? make_key(top1, row1) : 0ull;
+        best0 = row_ror_max<0x124>(row_ror_max<0x128>(best0));
+        best1 = row_ror_max<0x124>(row_ror_max<0x128>(best1));
         if (g == 0 && u < nc) {
             if (best0) atomicMax(&s.wgkey[c0 + u][0], best0);
             if (best1) atomicMax(&s.wgkey[c0 + u][1], best1);
         }
         // the keys stored next say that this workgroup's other stores of the iteration have landed
-        if (c0 + kTile >= s.ncol) __builtin_amdgcn_s_waitcnt(0);
+        if (c0 + kTile >= ncol) __builtin_amdgcn_s_waitcnt(0);
         lds_sync();
         TLA(27);
         pmark(p, s, tlast, kPrJCompute);
     }
     // this workgroup's stamped best token key of every joint column, one line per
     // workgroup; the duration keys from the ranks that own duration rows
-    if (threadIdx.x < 2 * s.ncol) {
+    if (threadIdx.x < 2 * ncol) {
         const int u = threadIdx.x >> 1, head = threadIdx.x & 1;
         const unsigned long long k = ((unsigned long long)stamp << kStampShift) | s.wgkey[u][head];
         const size_t par = stamp & 1;
@@ -1552,8 +1612,8 @@ __device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs
 // Each thread issues the loads of up to kL0 units before computing any.
 constexpr int kL0 = 3;
 __device__ __forceinline__ void lstm_layer0(const KParams &p, Ctl &s, const Lds &S, const Bufs &B, bool redundant,
-                                            int half) {
-    const int H = p.H, lgn = s.lgn, nl = s.nl;
+                                            int half, int nl, int lgn) {
+    const int H = p.H;
     const int n_work = (redundant ? H / 4 : s.own_lstm) << (lgn + 2);
     for (int base = 0; base < n_work; base += kL0 * kBlock) {
         float4 e[kL0], r[kL0];
@@ -1564,11 +1624,11 @@ __device__ __forceinline__ void lstm_layer0(const KParams &p, Ctl &s, const Lds 
             const int k = i >> (lgn + 2), u = (i >> 2) & ((1 << lgn) - 1);
             const int j = 4 * (redundant ? k : s.rank + k * s.P) + (i & 3);
             const bool ok = i < n_work && u < nl;
-            const int ul = s.lst[u < nl ? u : 0], b = s.b[ul], old = s.cur[ul] ^ 1;
-            const bool st = ok && !(s.flags[ul] & kFlagZeroHC);
-            e[q] = ld4(B.ep, ok ? (unsigned)(((size_t)s.pend[ul] * 4 * H + 4 * j) * 4) : kBad);
-            r[q] = ld4_coh(B.rx, st ? (unsigned)((rx_off(p, old, b) + 4 * j) * 4) : kBad);
-            c_prev[q] = ld1_coh(B.cx, st ? (unsigned)((cx_off(p, old, b) + j) * 4) : kBad);
+            const int2 row = *reinterpret_cast<const int2 *>(&s.lrow[u < nl ? u : 0]);
+            const bool st = ok && row.y >= 0;
+            e[q] = ld4(B.ep, ok ? (unsigned)(row.x + 16 * j) : kBad);
+            r[q] = ld4_coh(B.rx, st ? (unsigned)(4 * row.y + 16 * j) : kBad);
+            c_prev[q] = ld1_coh(B.cx, st ? (unsigned)(row.y + 4 * j) : kBad);
         }
 #pragma unroll
         for (int q = 0; q < kL0; ++q) {
@@ -1576,7 +1636,7 @@ __device__ __forceinline__ void lstm_layer0(const KParams &p, Ctl &s, const Lds 
             const int k = i >> (lgn + 2), u = (i >> 2) & ((1 << lgn) - 1), g = i & 3;
             if (i >= n_work || u >= nl) continue;
             const int tile = redundant ? k : s.rank + k * s.P, j = 4 * tile + g;
-            const int ul = s.lst[u], b = s.b[ul], cur = s.cur[ul];
+            const int2 row = *(reinterpret_cast<const int2 *>(&s.lrow[u]) + 1);
             float c_new, h_new;
             cell(e[q].x + r[q].x, e[q].y + r[q].y, e[q].z + r[q].z, e[q].w + r[q].w, c_prev[q], c_new, h_new);
             if (redundant) {   // straight into the layer-1 activation block
@@ -1587,8 +1647,8 @@ __device__ __forceinline__ void lstm_layer0(const KParams &p, Ctl &s, const Lds 
             }
             // owner of the tile (always, when only this workgroup's units are listed)
             if (!redundant || tile - udiv(tile, s.mag_p, s.P) * s.P == s.rank) {
-                st_coh(p.cx + cx_off(p, cur, b) + j, c_new);
-                st_coh(p.hs + hs_off(p, 0, b) + j, h_new);
+                st_coh(p.cx + (row.x >> 2) + j, c_new);
+                st_coh(p.hs + ((row.y & kRowMask) >> 2) + j, h_new);
             }
         }
     }
@@ -1620,8 +1680,9 @@ __device__ __forceinline__ void consume_layer(const KParams &p, Ctl &s, const Ld
     // pred rows) for one utterance u of the column tile
     const int layer = lc + 1, u = 4 * (lane >> 4) + (lane & 3), g = (lane >> 2) & 3;
     // this lane's utterance (a valid index for every lane; lanes u >= nc store nothing)
-    const int ul = s.lst[c0 + min(u, nc - 1)], b = s.b[ul], cur = s.cur[ul];
-    const bool zero = s.flags[ul] & kFlagZeroHC;
+    const int2 row = *(reinterpret_cast<const int2 *>(&s.lrow[c0 + min(u, nc - 1)]) + 1);
+    const int ul = row.y & kRowUl, cur = (row.y & kRowCur) ? 1 : 0;
+    const bool zero = row.y & kRowZero;
     // bias rows of the consumer tiles (LDS table): lane rows row0 .. row0+3 are
     // the pred rows, or the four gates of unit j = row0 / 4
     const float *btab = S.bias + kTile * lc * s.own_lstm;
@@ -1634,7 +1695,7 @@ __device__ __forceinline__ void consume_layer(const KParams &p, Ctl &s, const Ld
                       const int k = it - n_c;
                       if (lc == 0) {        // R_0: read by the layer-0 update of every workgroup (global)
                           const int row0 = (s.rank + k * s.P) * kTile + g * 4;
-                          st4_coh(B.rx, (unsigned)((rx_off(p, cur, b) + row0) * 4),
+                          st4_coh(B.rx, (unsigned)(4 * row.x + 4 * row0),
                                   make_float4(acc[0], acc[1], acc[2], acc[3]));
                       } else {              // R_lc: LDS state of this workgroup
                           *reinterpret_cast<float4 *>(st_at(p, S, lc, ul, k) + g * 4) =
@@ -1665,7 +1726,7 @@ __device__ __forceinline__ void consume_layer(const KParams &p, Ctl &s, const Ld
                        (acc[3] + r.w) + bias.w, c_prev, c_new, h_new);
                   st[kTile + g] = c_new;
                   st_coh(p.hx + hx_at(p, s.dom, layer, half, s.rank + it * s.P, c0 + u) + g, filled(h_new));
-                  st_coh(p.hs + hs_off(p, layer, b) + row0 / 4, h_new);
+                  st_coh(p.hs + (size_t)layer * p.n_utts * p.H + ((row.y & kRowMask) >> 2) + row0 / 4, h_new);
               });
 }
 
@@ -1688,17 +1749,17 @@ __device__ __forceinline__ void empty_h(const KParams &p, const Ctl &s, const Bu
 // previous step, whose half is emptied here.
 template <int WC>
 __device__ __forceinline__ void lstm_and_pred(const KParams &p, Ctl &s, const Bufs &B, const Lds &S, int half,
-                                              int n_prev, unsigned long long &tlast) {
+                                              int n_prev, int nl, int lgn, unsigned long long &tlast) {
     const int L = p.L;
-    const bool redundant = s.nl <= kSmallB && p.n_dom == 1;
-    lstm_layer0(p, s, S, B, redundant, half);
+    const bool redundant = nl <= kSmallB && p.n_dom == 1;
+    lstm_layer0(p, s, S, B, redundant, half, nl, lgn);
     empty_h(p, s, B, half ^ 1, n_prev);
     TLA(1);
     pmark(p, s, tlast, kPrL0);
     for (int lc = 0; lc < L; ++lc) {
         const bool local = lc == 0 && redundant;     // h_0' is in LDS already
-        for (int c0 = 0; c0 < s.nl; c0 += kTile) {
-            const int nc = min(kTile, s.nl - c0);
+        for (int c0 = 0; c0 < nl; c0 += kTile) {
+            const int nc = min(kTile, nl - c0);
             Act x = S.act[1];
             x.n = nc;
             // (redundant layer 0 wrote h_0' into the block itself.)  The block's last readers, the
@@ -1713,12 +1774,6 @@ __device__ __forceinline__ void lstm_and_pred(const KParams &p, Ctl &s, const Bu
         }
         pmark(p, s, tlast, lc == L - 1 ? kPrPred : kPrL1);
     }
-    for (int i = threadIdx.x; i < s.nl; i += kBlock) {   // the step is taken
-        const int ul = s.lst[i];
-        s.pend[ul] = -1;
-        s.flags[ul] &= ~kFlagZeroHC;
-        s.stp[ul] = 1;
-    }
 }
 
 // Apply the argmax results of iteration `stamp` to every utterance of the joint
@@ -1732,9 +1787,9 @@ __device__ __forceinline__ void lstm_and_pred(const KParams &p, Ctl &s, const Bu
 // data.  A rank cannot overwrite a key before every workgroup has read it: it
 // stores the same half again two iterations on, after the keys of the next.
 constexpr int kKeyRounds = 4;
-__device__ __forceinline__ void gather_keys(const KParams &p, Ctl &s, const Bufs &B, unsigned stamp) {
+__device__ __forceinline__ void gather_keys(const KParams &p, Ctl &s, const Bufs &B, unsigned stamp, int ncol) {
     lds_sync();   // this workgroup's key stores have read s.wgkey
-    const int P = s.P, nc = s.ncol, lane = threadIdx.x & (kWave - 1);
+    const int P = s.P, nc = ncol, lane = threadIdx.x & (kWave - 1);
     const int lgp = nc <= 2 ? 0 : 31 - __builtin_clz((unsigned)(nc - 1));   // log2 of the column pairs, rounded up
     const int pairs = 1 << lgp, cp = threadIdx.x & (pairs - 1), r0 = threadIdx.x >> lgp, step = kBlock >> lgp;
     const unsigned dom = (stamp & 1) * p.n_dom + s.dom;
@@ -1776,11 +1831,8 @@ __device__ __forceinline__ void gather_keys(const KParams &p, Ctl &s, const Bufs
         }
     }
     if (kd != 0ull) atomicMax(&s.wgkey[dc][1], kd);
-    for (int m = pairs; m < kWave; m <<= 1) {
-        const unsigned long long o0 = __shfl_xor(best0, m, kWave), o1 = __shfl_xor(best1, m, kWave);
-        best0 = o0 > best0 ? o0 : best0;
-        best1 = o1 > best1 ? o1 : best1;
-    }
+    best0 = lanes_max(best0, pairs);
+    best1 = lanes_max(best1, pairs);
     if (lane < pairs) {
         if (best0 != 0ull) atomicMax(&s.wgkey[2 * cp][0], best0);
         if (best1 != 0ull) atomicMax(&s.wgkey[2 * cp + 1][0], best1);
@@ -1788,113 +1840,110 @@ __device__ __forceinline__ void gather_keys(const KParams &p, Ctl &s, const Bufs
     lds_sync();
 }
 
-// One utterance per thread.  Its first decision is column i (frame t); while
-// the decision keeps the prediction output (a TDT blank; an EOU blank, <EOB>
+// One utterance per lane of wave 0.  Its first decision is column u.col (frame t);
+// while the decision keeps the prediction output (a TDT blank; an EOU blank, <EOB>
 // or special piece) and the next frame's column was evaluated, the walk goes
 // on with that column, one step per column, exactly as later iterations would.
-// CHAIN: spare columns were evaluated this iteration (otherwise sbase / sn are
-// stale and every utterance takes exactly one step).
-template <bool CHAIN>
-__device__ __forceinline__ void decide_steps(const KParams &p, Ctl &s, unsigned stamp) {
-    for (int i = threadIdx.x; i < s.nj; i += kBlock) {
-        const int ul = s.jst[i], b = s.b[ul];
-        const bool writer = ((s.wmask >> ul) & 1u) != 0u;
-        const int t0 = s.t[ul];
-        int col = i;
-        while (true) {
-            const unsigned long long kt = s.wgkey[col][0], kd = s.wgkey[col][1];
-            if (key_stamp(kt) != stamp || (p.Dn > 0 && key_stamp(kd) != stamp)) {
-                __hip_atomic_store(p.status, PK_ERR_DEVICE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s.t[ul] = s.T[ul];
-                break;
-            }
-            const int tok = key_index(kt);
-            const int di = p.Dn > 0 ? key_index(kd) : -1;
-            const int step = s.steps[ul]++;
-            if (p.logits && step < p.logit_steps) {
-                const int q = atomicAdd(&s.tq_n, 1);
-                s.tq_col[q] = col;
-                s.tq_b[q] = b;
-                s.tq_step[q] = step;
-            }
-            if (writer && p.trace) {
-                if (step < p.trace_cap) {
-                    p.trace[((size_t)b * p.trace_cap + step) * 2] = tok;
-                    p.trace[((size_t)b * p.trace_cap + step) * 2 + 1] = di;
-                } else {
-                    s.flags[ul] |= kFlagTraceOverflow;
-                }
-            }
-            bool keep = false;   // the prediction output stays: the next frame may follow at once
-            if (p.kind == PK_KIND_TDT) {
-                const int dur = p.n_dur > 0 ? s.dur[di] : di;
-                const int adv = dur > 1 ? dur : 1;
-                if (tok == p.blank) {
-                    s.t[ul] += adv;
-                    s.sym[ul] = 0;
-                    keep = true;
-                } else {
-                    const int n = s.ntok[ul]++;
-                    if (writer) {
-                        if (n < p.token_cap) p.tokens[(size_t)b * p.token_cap + n] = tok;
-                        else s.flags[ul] |= kFlagTokOverflow;
-                    }
-                    s.pend[ul] = tok;
-                    s.cur[ul] ^= 1;
-                    s.sym[ul] += 1;
-                    if (dur > 0 || s.sym[ul] >= p.max_sym) {
-                        s.t[ul] += adv;
-                        s.sym[ul] = 0;
-                    }
-                }
-            } else {
-                const int max_syms = p.max_sym > 1 ? p.max_sym : 1;
-                bool frame_done = false;
-                if (tok == p.blank || tok == p.eob) {
-                    frame_done = true;
-                    keep = true;
-                } else if (tok == p.eou) {
-                    const int total = s.tbase[ul] + s.ntok[ul];
-                    if (total > s.segst[ul]) {
-                        const int ns = s.nseg[ul]++;
-                        if (writer) {
-                            if (p.segs && ns < p.seg_cap) p.segs[(size_t)b * p.seg_cap + ns] = total;
-                            else s.flags[ul] |= kFlagSegOverflow;
-                        }
-                        s.segst[ul] = total;
-                    }
-                    s.flags[ul] |= kFlagZeroHC;
-                    s.pend[ul] = p.blank;
-                    s.cur[ul] ^= 1;
-                    s.last[ul] = p.blank;
-                    frame_done = true;
-                } else if (tok >= 0 && tok < p.n_special && p.special[tok]) {
-                    frame_done = true;
-                    keep = true;
-                } else {
-                    const int n = s.ntok[ul]++;
-                    if (writer) {
-                        if (n < p.token_cap) p.tokens[(size_t)b * p.token_cap + n] = tok;
-                        else s.flags[ul] |= kFlagTokOverflow;
-                    }
-                    s.pend[ul] = tok;
-                    s.cur[ul] ^= 1;
-                    s.last[ul] = tok;
-                    s.sym[ul] += 1;
-                    if (s.sym[ul] >= max_syms) frame_done = true;
-                }
-                if (frame_done) {          // the next frame starts with sym = 0 (src/parakeet_eou.cpp:269)
-                    s.t[ul] += 1;
-                    if (s.t[ul] < s.T[ul]) s.sym[ul] = 0;
-                }
-            }
-            // the next decision's frame offset from t0, if its column was evaluated
-            s.brun[ul] = keep ? 1 : 0;
-            if (!CHAIN || !keep || s.t[ul] >= s.T[ul]) break;
-            const int o = s.t[ul] - t0;
-            if (o > s.sn[i]) break;
-            col = s.sbase[i] + o - 1;
+__device__ __forceinline__ void decide_steps(const KParams &p, Ctl &s, Utt &u, unsigned stamp) {
+    const int ul = threadIdx.x;
+    if (ul >= s.n || u.t >= u.T) return;
+    const int b = s.b[ul];
+    const bool writer = ((s.wmask >> ul) & 1u) != 0u;
+    const int t0 = u.t;
+    int col = u.col;
+    while (true) {
+        const unsigned long long kt = s.wgkey[col][0], kd = s.wgkey[col][1];
+        if (key_stamp(kt) != stamp || (p.Dn > 0 && key_stamp(kd) != stamp)) {
+            __hip_atomic_store(p.status, PK_ERR_DEVICE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            u.t = u.T;
+            break;
         }
+        const int tok = key_index(kt);
+        const int di = p.Dn > 0 ? key_index(kd) : -1;
+        const int step = u.steps++;
+        if (p.logits && step < p.logit_steps) {
+            const int q = atomicAdd(&s.tq_n, 1);
+            s.tq_col[q] = col;
+            s.tq_b[q] = b;
+            s.tq_step[q] = step;
+        }
+        if (writer && p.trace) {
+            if (step < p.trace_cap) {
+                p.trace[((size_t)b * p.trace_cap + step) * 2] = tok;
+                p.trace[((size_t)b * p.trace_cap + step) * 2 + 1] = di;
+            } else {
+                u.flags |= kFlagTraceOverflow;
+            }
+        }
+        bool keep = false;   // the prediction output stays: the next frame may follow at once
+        if (p.kind == PK_KIND_TDT) {
+            const int dur = p.n_dur > 0 ? s.dur[di] : di;
+            const int adv = dur > 1 ? dur : 1;
+            if (tok == p.blank) {
+                u.t += adv;
+                u.sym = 0;
+                keep = true;
+            } else {
+                const int n = u.ntok++;
+                if (writer) {
+                    if (n < p.token_cap) p.tokens[(size_t)b * p.token_cap + n] = tok;
+                    else u.flags |= kFlagTokOverflow;
+                }
+                u.pend = tok;
+                u.cur ^= 1;
+                u.sym += 1;
+                if (dur > 0 || u.sym >= p.max_sym) {
+                    u.t += adv;
+                    u.sym = 0;
+                }
+            }
+        } else {
+            const int max_syms = p.max_sym > 1 ? p.max_sym : 1;
+            bool frame_done = false;
+            if (tok == p.blank || tok == p.eob) {
+                frame_done = true;
+                keep = true;
+            } else if (tok == p.eou) {
+                const int total = s.tbase[ul] + u.ntok;
+                if (total > s.segst[ul]) {
+                    const int ns = s.nseg[ul]++;
+                    if (writer) {
+                        if (p.segs && ns < p.seg_cap) p.segs[(size_t)b * p.seg_cap + ns] = total;
+                        else u.flags |= kFlagSegOverflow;
+                    }
+                    s.segst[ul] = total;
+                }
+                u.flags |= kFlagZeroHC;
+                u.pend = p.blank;
+                u.cur ^= 1;
+                s.last[ul] = p.blank;
+                frame_done = true;
+            } else if (tok >= 0 && tok < p.n_special && p.special[tok]) {
+                frame_done = true;
+                keep = true;
+            } else {
+                const int n = u.ntok++;
+                if (writer) {
+                    if (n < p.token_cap) p.tokens[(size_t)b * p.token_cap + n] = tok;
+                    else u.flags |= kFlagTokOverflow;
+                }
+                u.pend = tok;
+                u.cur ^= 1;
+                s.last[ul] = tok;
+                u.sym += 1;
+                if (u.sym >= max_syms) frame_done = true;
+            }
+            if (frame_done) {          // the next frame starts with sym = 0 (src/parakeet_eou.cpp:269)
+                u.t += 1;
+                if (u.t < u.T) u.sym = 0;
+            }
+        }
+        // the next decision's frame offset from t0, if its column was evaluated
+        u.keep = keep ? 1 : 0;
+        if (!keep || u.t >= u.T) break;
+        const int o = u.t - t0;
+        if (o > u.sn) break;
+        col = u.sbase + o - 1;
     }
 }
 
@@ -1916,10 +1965,12 @@ __device__ __forceinline__ void tap_copy(const KParams &p, Ctl &s) {
     if (threadIdx.x == 0) s.tq_n = 0;
 }
 
-__device__ __forceinline__ void decide(const KParams &p, Ctl &s, unsigned stamp) {
-    if (s.ncol > s.nj) decide_steps<true>(p, s, stamp);
-    else decide_steps<false>(p, s, stamp);
-    if (p.logits) tap_copy(p, s);
+__device__ __forceinline__ void decide(const KParams &p, Ctl &s, Utt &u, unsigned stamp) {
+    if (threadIdx.x < kWave) decide_steps(p, s, u, stamp);
+    if (p.logits) {
+        lds_sync();
+        tap_copy(p, s);
+    }
 }
 
 // Co-residency of an ordinary dispatch.  The loop's barriers need every
@@ -2046,31 +2097,29 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
     }
     if (threadIdx.x < PK_MAX_DURATIONS) s.dur[threadIdx.x] = threadIdx.x < p.n_dur ? p.durations[threadIdx.x] : 0;
     __syncthreads();
-    for (int ul = threadIdx.x; ul < s.n; ul += kBlock) {
-        const int b = p.dom_list[s.dom * kDomCap + ul];
+    Utt u{};
+    u.pend = -1;
+    if (threadIdx.x < s.n) {
+        const int ul = threadIdx.x, b = p.dom_list[s.dom * kDomCap + ul];
         const int slot = p.slot[b];
         const int *ctrl = p.slot_ctrl + (size_t)slot * PK_CTRL_N;
         const bool init = ctrl[PK_CTRL_INIT] != 0 && !(p.reset && p.reset[b]);
+        u.T = p.T[b];
+        u.cur = init ? 0 : 1;   // (a fresh utterance's first step is pending)
+        u.sym = init ? ctrl[PK_CTRL_SYM] : 0;
+        if (p.kind == PK_KIND_EOU && u.T > 0) u.sym = 0;   // reset per frame (src/parakeet_eou.cpp:269)
+        const int carry = init ? ctrl[PK_CTRL_CARRY] : 0;
+        u.pend = init ? -1 : p.blank;
+        u.flags = init ? 0 : kFlagZeroHC;
+        if (p.kind == PK_KIND_TDT) u.t = carry > 0 ? min(carry, u.T) : 0;
         s.b[ul] = b;
-        s.T[ul] = p.T[b];
-        s.erow[ul] = p.encp_row[b];
+        s.erow[ul] = (unsigned)((size_t)p.encp_row[b] * J * 4);
         s.bbias[ul] = p.blank_bias ? p.blank_bias[b] : 0.0f;
         s.tbase[ul] = p.tokens_base ? p.tokens_base[b] : 0;
-        s.ntok[ul] = 0;
-        s.steps[ul] = 0;
         s.nseg[ul] = 0;
-        s.cur[ul] = init ? 0 : 1;   // (a fresh utterance's first step is pending)
-        s.stp[ul] = 0;
-        s.sym[ul] = init ? ctrl[PK_CTRL_SYM] : 0;
-        if (p.kind == PK_KIND_EOU && s.T[ul] > 0) s.sym[ul] = 0;   // reset per frame (src/parakeet_eou.cpp:269)
         s.last[ul] = init ? ctrl[PK_CTRL_LAST] : -1;
         s.segst[ul] = init ? ctrl[PK_CTRL_SEGSTART] : 0;
-        const int carry = init ? ctrl[PK_CTRL_CARRY] : 0;
-        s.pend[ul] = init ? -1 : p.blank;
-        s.flags[ul] = init ? 0 : kFlagZeroHC;
-        s.brun[ul] = 0;
-        if (p.kind == PK_KIND_TDT) s.t[ul] = carry > 0 ? min(carry, s.T[ul]) : 0;
-        else s.t[ul] = 0;
+        s.mark[ul] = init ? 0 : 1;
     }
     __syncthreads();
     // copy c_0, R_0 and pp of this workgroup's utterances from their slots into the
@@ -2078,7 +2127,7 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
     // the words the loop waits for: the other half of pp, this workgroup's tiles of h
     for (int ul = s.rank; ul < s.n; ul += s.P) {
         const int b = s.b[ul], slot = p.slot[b];
-        const bool fresh = s.flags[ul] & kFlagZeroHC;
+        const bool fresh = s.mark[ul] != 0;
         const float *src_c = p.slot_c + (size_t)slot * L * H, *src_r = p.slot_r + (size_t)slot * L * 4 * H,
                     *src_p = p.slot_pp + (size_t)slot * J;
         const int nq = fresh ? 0 : (H + 4 * H + J) / 4;
@@ -2123,14 +2172,16 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
         cache_matrix(p.w_pred, s.rank, s.P, wcache);
         cache_matrix(p.w_out, s.rank, s.P, wcache);
     }
-    build_lists(s, p.spec != 0);
+    build_lists(p, s, u);
     bool ok = dom_sync(p, s, epoch);
 
     unsigned iter = 0;
     int half = 0, n_prev = 0;   // half of hx of the next LSTM step; list length of the previous one
     unsigned long long tlast = __builtin_amdgcn_s_memrealtime();
     while (ok) {
-        if (s.nl == 0 && s.nj == 0) break;
+        const int nl = __builtin_amdgcn_readfirstlane(s.cnt.x), nj = __builtin_amdgcn_readfirstlane(s.cnt.y),
+                  ncol = __builtin_amdgcn_readfirstlane(s.cnt.z), lgn = __builtin_amdgcn_readfirstlane(s.cnt.w);
+        if (nl == 0 && nj == 0) break;
         if ((int)iter >= p.max_iter) {
             if (threadIdx.x == 0)
                 __hip_atomic_store(p.status, PK_ERR_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2148,25 +2199,30 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
         }
 #endif
         float4 epre[kStageMax];
-        if (s.nj > 0) encp_prefetch(p, s, B, epre);
-        if (s.nl > 0) {
-            lstm_and_pred<WC>(p, s, B, S, half, n_prev, tlast);
+        if (nj > 0) encp_prefetch(p, s, B, ncol, epre);
+        if (nl > 0) {
+            lstm_and_pred<WC>(p, s, B, S, half, n_prev, nl, lgn, tlast);
             half ^= 1;
-            n_prev = s.nl;
+            n_prev = nl;
+            if (u.pend >= 0) {   // the step is taken
+                u.pend = -1;
+                u.flags &= ~kFlagZeroHC;
+                u.stp = 1;
+            }
         }
-        if (s.nj > 0) {
-            joint_phase<WC>(p, s, B, S, iter, epre, tlast);
-            gather_keys(p, s, B, iter);
+        if (nj > 0) {
+            joint_phase<WC>(p, s, B, S, iter, ncol, epre, tlast);
+            gather_keys(p, s, B, iter, ncol);
             TLA(29);
             pmark(p, s, tlast, kPrKeys);
             if (!s.ok) {   // (behind the gather's barrier: the same in every wave)
                 ok = false;
                 break;
             }
-            decide(p, s, iter);
+            decide(p, s, u, iter);
         }
-        lds_sync();
-        build_lists(s, p.spec != 0);
+        if (nj == 0) lds_sync();   // (behind the keys' barrier otherwise)
+        build_lists(p, s, u);
         TLA(31);
         pmark(p, s, tlast, kPrDecide);
     }
@@ -2175,6 +2231,10 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
     if (p.prof && wg == 0 && threadIdx.x < kWaves * kTl) p.prof[kPrN + threadIdx.x] = tl_sum()[threadIdx.x];
     if (p.prof && wg == 0 && threadIdx.x < kTl) p.prof[kPrN + kWaves * kTl + threadIdx.x] = tl_ctl()[2 + threadIdx.x];
 #endif
+    if (threadIdx.x < s.n) {
+        s.cur[threadIdx.x] = u.cur;
+        s.mark[threadIdx.x] = u.stp;
+    }
     __builtin_amdgcn_s_waitcnt(0);   // this workgroup's state stores have landed
     __syncthreads();
     if (!ok || !s.ok) return;
@@ -2221,30 +2281,29 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
                 dst = p.slot_pp + (size_t)p.slot[s.b[ul]] * J + t * kTile + g * 4;
                 x = (p.ppx - p.hs) + (long long)ppx_at(p, s.dom, s.cur[ul], t, ul) + g * 4;
             }
-            if (s.stp[ul]) *reinterpret_cast<float4 *>(dst) = ld4_coh(bx, (unsigned)(x * 4));
+            if (s.mark[ul]) *reinterpret_cast<float4 *>(dst) = ld4_coh(bx, (unsigned)(x * 4));
         }
     }
-    for (int ul = s.rank; ul < s.n; ul += s.P) {
-        const int b = s.b[ul], slot = p.slot[b];
-        if (threadIdx.x < PK_CTRL_N) {   // the slot's control words (and the caller's copy)
-            const int k = threadIdx.x;
+    if (threadIdx.x < s.n && ((s.wmask >> threadIdx.x) & 1u) != 0u) {   // outputs and control words
+        const int ul = threadIdx.x, b = s.b[ul];
+        int *ctrl = p.slot_ctrl + (size_t)p.slot[b] * PK_CTRL_N;
+#pragma unroll
+        for (int k = 0; k < PK_CTRL_N; ++k) {
             const int v = k == PK_CTRL_INIT ? 1
-                        : k == PK_CTRL_SYM ? s.sym[ul]
-                        : k == PK_CTRL_CARRY ? ((p.kind == PK_KIND_TDT) ? max(0, s.t[ul] - s.T[ul]) : 0)
+                        : k == PK_CTRL_SYM ? u.sym
+                        : k == PK_CTRL_CARRY ? ((p.kind == PK_KIND_TDT) ? max(0, u.t - u.T) : 0)
                         : k == PK_CTRL_LAST ? s.last[ul]
                         : k == PK_CTRL_SEGSTART ? s.segst[ul] : 0;
-            p.slot_ctrl[(size_t)slot * PK_CTRL_N + k] = v;
+            ctrl[k] = v;
             if (p.ctrl_out) p.ctrl_out[(size_t)b * PK_CTRL_N + k] = v;
         }
-        if (threadIdx.x == 0) {
-            p.n_tokens[b] = s.ntok[ul];
-            p.steps[b] = s.steps[ul];
-            if (p.n_segs) p.n_segs[b] = s.nseg[ul];
-            if (s.flags[ul] & (kFlagTokOverflow | kFlagSegOverflow))
-                __hip_atomic_store(p.status + 2, PK_ERR_OVERFLOW, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (s.flags[ul] & kFlagTraceOverflow)
-                __hip_atomic_store(p.status + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        p.n_tokens[b] = u.ntok;
+        p.steps[b] = u.steps;
+        if (p.n_segs) p.n_segs[b] = s.nseg[ul];
+        if (u.flags & (kFlagTokOverflow | kFlagSegOverflow))
+            __hip_atomic_store(p.status + 2, PK_ERR_OVERFLOW, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (u.flags & kFlagTraceOverflow)
+            __hip_atomic_store(p.status + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (threadIdx.x == 0) atomicMax(p.status + 1, (int)iter);
 }
