@@ -75,10 +75,15 @@ using pkdev::kWave;
 using pkdev::kWaves;
 
 constexpr int kMaxBatch = PK_MAX_BATCH;
-// host outputs up to this size come back whole with the counters (one stream wait per call)
+// host outputs up to this size are written by the kernel straight into pinned memory: the call waits
+// for the stream once and copies nothing back (one EOU-120m session, two-frame chunks, frames and
+// results in host memory: 95 -> 88 us per call, with the frames and the descriptor block going up in
+// one copy; seven TDT-0.6b utterances with tapped logits -3 %)
 constexpr size_t kEagerCopyBytes = 256 << 10;
 // host frames up to this size go up through a pinned staging block of the decoder
 constexpr size_t kPinnedFrames = 64ull << 20;
+// host frames up to this size go up in one copy with the descriptor block
+constexpr size_t kJoinedFrames = 1 << 20;
 // windows shorter than this many frames do not fill the LDS weight cache
 constexpr int kCacheMinFrames = 16;
 // enc_proj over at most this many rows runs the narrow kernel (one wave per 16x16 block;
@@ -1241,17 +1246,23 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
         return fail(PK_ERR_UNSUPPORTED, "window too long for the iteration stamp of one launch");
     const int D = dec->desc.d_enc, J = p.J, L = p.L, H = p.H;
     int rc;
-    // encoder frames: device pointer as given, or packed host rows uploaded
+    // encoder frames: device pointer as given, or packed host rows uploaded (a few rows together
+    // with the descriptor block below, in one copy)
     const float *enc = bt->enc;
+    const size_t desc_room = 36 * (size_t)m + 4 * (size_t)dec->nwg * (kDomCap + 4) + 64;   // at least desc_bytes
+    bool joined = false;
     if (enc_host && rows > 0) {
-        if ((rc = dec->d_enc.ensure((size_t)rows * D * 4))) return rc;
+        const bool few = (size_t)rows * D * 4 <= kJoinedFrames;
+        if ((rc = dec->d_enc.ensure((size_t)rows * D * 4 + (few ? desc_room : 0)))) return rc;
         // up to kPinnedFrames bytes the rows are gathered into pinned memory and go up in one
         // asynchronous copy; beyond, one copy from the caller's (pageable) memory per run of
         // utterances whose source rows follow each other.  The device rows are packed in
         // utterance order.
         const size_t fbytes = (size_t)rows * D * 4;
         float *pin = nullptr;
-        if (fbytes <= kPinnedFrames && dec->h_frames.ensure(fbytes) == 0) pin = dec->h_frames.as<float>();
+        if (fbytes <= kPinnedFrames && dec->h_frames.ensure(fbytes + (few ? desc_room : 0)) == 0)
+            pin = dec->h_frames.as<float>();
+        joined = few && pin;
         for (int i = 0; i < m;) {
             int j = i + 1;
             long long end = src_row[i] + T[i];
@@ -1268,7 +1279,7 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
                                        hipMemcpyHostToDevice, dec->stream));
             i = j;
         }
-        if (pin) HIP_TRY(hipMemcpyAsync(dec->d_enc.p, pin, fbytes, hipMemcpyHostToDevice, dec->stream));
+        if (pin && !joined) HIP_TRY(hipMemcpyAsync(dec->d_enc.p, pin, fbytes, hipMemcpyHostToDevice, dec->stream));
         enc = dec->d_enc.as<float>();
         src_row = dst_row;
     }
@@ -1285,9 +1296,13 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
                                               pl.wg_dom.size() + pl.wg_rank.size() + pl.dom_wg.size();
     const size_t desc_bytes = n64 * 8 + n32 * 4;
     void *d_desc = nullptr;
-    if ((rc = cs.get(dec->d_desc, desc_bytes, &d_desc))) return rc;
     uint8_t *hd;
-    if (16 + desc_bytes <= dec->pin_cnt) {
+    const size_t fbytes = (size_t)rows * D * 4;
+    if (joined) d_desc = static_cast<uint8_t *>(dec->d_enc.p) + fbytes;
+    else if ((rc = cs.get(dec->d_desc, desc_bytes, &d_desc))) return rc;
+    if (joined) {   // behind the frames (desc_bytes <= desc_room: at most nwg domains of kDomCap)
+        hd = dec->h_frames.as<uint8_t>() + fbytes;
+    } else if (16 + desc_bytes <= dec->pin_cnt) {
         hd = dec->h_pin.as<uint8_t>() + 16;
     } else {
         dec->h_desc.resize(desc_bytes);
@@ -1312,7 +1327,10 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
     const int *d_wg_dom = reinterpret_cast<const int *>(put(pl.wg_dom.data(), 4 * pl.wg_dom.size()));
     const int *d_wg_rank = reinterpret_cast<const int *>(put(pl.wg_rank.data(), 4 * pl.wg_rank.size()));
     const int *d_dom_wg = reinterpret_cast<const int *>(put(pl.dom_wg.data(), 4 * pl.dom_wg.size()));
-    HIP_TRY(hipMemcpyAsync(d_desc, hd, desc_bytes, hipMemcpyHostToDevice, dec->stream));
+    if (joined)
+        HIP_TRY(hipMemcpyAsync(dec->d_enc.p, dec->h_frames.p, fbytes + desc_bytes, hipMemcpyHostToDevice, dec->stream));
+    else
+        HIP_TRY(hipMemcpyAsync(d_desc, hd, desc_bytes, hipMemcpyHostToDevice, dec->stream));
 
     // column capacity of the argmax keys, row capacities of the exchange buffers (powers of two;
     // h rows at least 8, a whole 128-byte line per unit tile)
@@ -1361,11 +1379,14 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
     const size_t lrow = (size_t)lsteps * p.Vo;   // tapped floats per utterance
     int *o_tok, *o_ntok, *o_steps, *o_seg = nullptr, *o_nseg = nullptr, *o_trace = nullptr, *o_ctrl = nullptr;
     float *o_logits = nullptr;
+    // host outputs of up to kEagerCopyBytes: the kernel writes them (each word once) straight into
+    // pinned memory and the call copies nothing back; larger ones go through device staging
+    const size_t out_words = (size_t)m * tcap + 3 * (size_t)m + (size_t)m * scap + (size_t)m * trcap * 2 +
+                             (size_t)m * PK_CTRL_N + (size_t)m * lrow;
+    const bool eager = host && (out_words - (3 + PK_CTRL_N) * (size_t)m) * 4 <= kEagerCopyBytes;
     if (host) {
-        const size_t need = ((size_t)m * tcap + 3 * (size_t)m + (size_t)m * scap + (size_t)m * trcap * 2 +
-                             (size_t)m * PK_CTRL_N + (size_t)m * lrow) * 4 + 64;
-        if ((rc = dec->d_out.ensure(need))) return rc;
-        int *o = dec->d_out.as<int>();
+        if ((rc = eager ? dec->h_out.ensure(std::max(out_words * 4, kEagerCopyBytes)) : dec->d_out.ensure(out_words * 4 + 64))) return rc;
+        int *o = eager ? dec->h_out.as<int>() : dec->d_out.as<int>();
         o_tok = o; o += (size_t)m * tcap;
         o_ntok = o; o += m;
         o_steps = o; o += m;
@@ -1514,26 +1535,13 @@ relaunch:
     int *status = dec->h_pin.as<int>();   // read after the stream synchronisation below
     HIP_TRY(hipMemcpyAsync(status, p.status, 4 * sizeof(int), hipMemcpyDeviceToHost, dec->stream));
     if (host) {
-        // The device staging is one block: tokens | n_tokens, steps, n_segments | segments |
-        // trace | control words.  Up to kEagerCopyBytes of rows it comes back whole in one
-        // copy, so the call waits for the stream once.  Larger outputs copy the counters and
-        // control words first, then only each row's filled prefix.
-        const size_t tb = (size_t)m * tcap * 4, sb_all = (size_t)m * scap * 4,
-                     rb = o_trace ? (size_t)m * trcap * 8 : 0, cb = o_ctrl ? (size_t)m * PK_CTRL_N * 4 : 0;
-        const bool eager = tb + sb_all + rb <= kEagerCopyBytes;
+        // Eager outputs are in pinned memory.  Larger ones copy the counters and control words
+        // first, then only each row's filled prefix.
+        const size_t cb = o_ctrl ? (size_t)m * PK_CTRL_N * 4 : 0;
         std::vector<int> cnt_v;
-        int *cnt, *e_tok, *e_seg, *e_tr;
-        int32_t *s_ctrl;
-        if (eager) {
-            const size_t whole = tb + 12 * (size_t)m + sb_all + rb + cb;
-            if ((rc = dec->h_out.ensure(std::max<size_t>(whole, 64)))) return rc;
-            HIP_TRY(hipMemcpyAsync(dec->h_out.p, o_tok, whole, hipMemcpyDeviceToHost, dec->stream));
-            e_tok = dec->h_out.as<int>();
-            cnt = e_tok + tb / 4;
-            e_seg = cnt + 3 * (size_t)m;
-            e_tr = e_seg + sb_all / 4;
-            s_ctrl = e_tr + rb / 4;
-        } else {
+        int *cnt = o_ntok, *e_tok = o_tok, *e_seg = o_seg, *e_tr = o_trace;
+        int32_t *s_ctrl = o_ctrl;
+        if (!eager) {
             if (dec->pin_cnt + 12 * (size_t)m <= dec->h_pin.n) {   // (m <= n_slots: slots are distinct)
                 cnt = reinterpret_cast<int *>(dec->h_pin.as<uint8_t>() + dec->pin_cnt);
             } else {
@@ -1588,10 +1596,13 @@ relaunch:
         if (o_ctrl)
             for (int i = 0; i < m; ++i)
                 memcpy(bt->ctrl_out + (size_t)map[i] * PK_CTRL_N, s_ctrl + (size_t)i * PK_CTRL_N, PK_CTRL_N * 4);
-        if (o_logits)   // debug tap: straight into the caller's rows (utterance order may differ)
-            for (int i = 0; i < m; ++i)
-                HIP_TRY(hipMemcpy(bt->logits + (size_t)map[i] * lrow, o_logits + (size_t)i * lrow, lrow * 4,
-                                  hipMemcpyDeviceToHost));
+        if (o_logits)   // debug tap: the rows of the steps taken (utterance order may differ)
+            for (int i = 0; i < m; ++i) {
+                const size_t taken = (size_t)std::min(c_steps[i], lsteps) * p.Vo * 4;
+                float *dst = bt->logits + (size_t)map[i] * lrow;
+                if (eager) memcpy(dst, o_logits + (size_t)i * lrow, taken);
+                else if (taken > 0) HIP_TRY(hipMemcpy(dst, o_logits + (size_t)i * lrow, taken, hipMemcpyDeviceToHost));
+            }
         for (int i = 0; i < m; ++i) {
             const int u = map[i];
             bt->n_tokens[u] = c_tok[i];

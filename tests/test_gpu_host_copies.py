@@ -1,0 +1,70 @@
+"""Host-memory calls around the sizes where their copies change: frames up with the descriptor block in
+one copy up to 1 MiB, outputs written straight into pinned memory up to 256 KiB (tokens, segments, trace
+and tapped logits together).  On either side of each line the results equal those of the same windows
+decoded from device frames with another split of the outputs, bit for bit, and the logit rows of steps an
+utterance does not reach stay untouched."""
+import numpy as np
+import pytest
+
+from conftest import small_eou, small_tdt
+from parity import check_window
+
+pytestmark = pytest.mark.gpu
+
+LINE_FRAMES, LINE_OUT = 1 << 20, 256 << 10
+
+
+def _equal(a, b):
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        assert x["steps"] == y["steps"]
+        for k in ("tokens", "segments", "ctrl"):
+            assert np.array_equal(x[k], y[k]), k
+
+
+@pytest.mark.parametrize("kind", ["tdt", "eou"])
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+def test_frames_line(tmp_path, kind, extra):
+    import torch
+    from parakeet_amd import gguf, pk, synth
+    import oracle
+    path = str(tmp_path / "d.gguf")
+    (small_tdt if kind == "tdt" else small_eou)(path)
+    om = oracle.OracleModel.from_gguf(path, gguf)
+    dev = pk.Decoder.from_gguf(path, n_slots=64)
+    D = dev.info.D
+    rows = LINE_FRAMES // (4 * D) + extra
+    T = [rows // 32] * 31
+    T.append(rows - sum(T))
+    encs = [synth.encoder_frames(40 + u, t, D) for u, t in enumerate(T)]
+    print(f"{kind}: {rows} frames of {4 * D} bytes", flush=True)
+    a = dev.decode(encs, slots=list(range(32)), trace=True)
+    flat = torch.from_numpy(np.concatenate(encs)).cuda()
+    torch.cuda.synchronize()
+    first = np.concatenate([[0], np.cumsum(T)[:-1]])
+    b = dev.decode_device_frames(flat.data_ptr(), first, T, slots=list(range(32, 64)))
+    _equal(a, b)
+    check_window(om, dev, 0, encs[0], a[0], om.new_state(), dev.info.max_symbols)
+    dev.close()
+
+
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+def test_outputs_line(tmp_path, extra):
+    from parakeet_amd import pk, synth
+    path = str(tmp_path / "d.gguf")
+    small_tdt(path)
+    dev = pk.Decoder.from_gguf(path, n_slots=8)
+    n, Vo = 4, dev.info.Vo
+    encs = [synth.encoder_frames(60 + u, 3 + u, dev.info.D) for u in range(n)]
+    steps = 64                                # more than any of the windows takes
+    # words per utterance: tokens, segments (one more), logits
+    cap = (LINE_OUT // 4 // n - 1 - steps * Vo) // 2 + extra
+    print(f"token capacity {cap}", flush=True)
+    a = dev.decode(encs, slots=[0, 1, 2, 3], token_cap=cap, logit_steps=steps)
+    b = dev.decode(encs, slots=[4, 5, 6, 7])
+    _equal(a, b)
+    for x in a:
+        assert 0 < x["steps"] < steps
+        assert not np.isnan(x["logits"][:x["steps"]]).any()
+        assert np.isnan(x["logits"][x["steps"]:]).all()
+    dev.close()
