@@ -25,8 +25,7 @@ def _equal(a, b):
 @pytest.mark.parametrize("kind", ["tdt", "eou"])
 @pytest.mark.parametrize("extra", [-1, 0, 1])
 def test_frames_line(tmp_path, kind, extra):
-    import torch
-    from parakeet_amd import gguf, pk, synth
+    from parakeet_amd import gguf, hipmem, pk, synth
     import oracle
     path = str(tmp_path / "d.gguf")
     (small_tdt if kind == "tdt" else small_eou)(path)
@@ -39,12 +38,12 @@ def test_frames_line(tmp_path, kind, extra):
     encs = [synth.encoder_frames(40 + u, t, D) for u, t in enumerate(T)]
     print(f"{kind}: {rows} frames of {4 * D} bytes", flush=True)
     a = dev.decode(encs, slots=list(range(32)), trace=True)
-    flat = torch.from_numpy(np.concatenate(encs)).cuda()
-    torch.cuda.synchronize()
+    flat = hipmem.DeviceArray.from_numpy(np.concatenate(encs))
     first = np.concatenate([[0], np.cumsum(T)[:-1]])
-    b = dev.decode_device_frames(flat.data_ptr(), first, T, slots=list(range(32, 64)))
+    b = dev.decode_device_frames(flat.ptr, first, T, slots=list(range(32, 64)))
     _equal(a, b)
     check_window(om, dev, 0, encs[0], a[0], om.new_state(), dev.info.max_symbols)
+    flat.free()
     dev.close()
 
 
