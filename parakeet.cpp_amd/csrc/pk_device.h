@@ -273,6 +273,20 @@ __device__ __forceinline__ u64 lanes_max(u64 v, int step) {
     return a > b ? a : b;
 }
 
+// Inclusive prefix sum over the wave: shifts inside a DPP row, then the rows' last lanes passed on.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int v) {
+    return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ int wave_scan(int v) {
+    v = dpp_add<0x111, 0xF>(v);   // row_shr:1
+    v = dpp_add<0x112, 0xF>(v);
+    v = dpp_add<0x114, 0xF>(v);
+    v = dpp_add<0x118, 0xF>(v);
+    v = dpp_add<0x142, 0xA>(v);   // row_bcast:15 into rows 1 and 3
+    return dpp_add<0x143, 0xC>(v);   // row_bcast:31 into rows 2 and 3
+}
+
 // Staged activation block: 16 utterance rows of K values as f16 (hi, lo).
 // Only rows 0 .. n-1 are staged; product columns n .. 15 are not used.
 struct Act {
@@ -707,7 +721,8 @@ struct Utt {
 
 struct Ctl {                      // per-workgroup state of its domain
     // the lists of an iteration, as the byte offsets their readers need
-    int4 cnt;                     // LSTM list length, joint list length, joint columns, log2 of the first, rounded up
+    int4 cnt;                     // LSTM list length (-1: the launch ends, see ok), joint list length, joint
+                                  // columns, log2 of the first, rounded up
     // LSTM list row: E' row of the pending token; c_0 row of the old state (-1: zero state) and of the
     // new one; h row | parity << 6 | zero state << 5 | domain utterance
     int4 lrow[kDomCap];
@@ -826,16 +841,13 @@ __device__ __forceinline__ void build_lists(const KParams &p, Ctl &s, Utt &u) {
             const int ne = __popcll(be), ie = __popcll(be & below);
             int q = 0;
             if (fe) {
-                q = spare / ne + (ie < spare % ne ? 1 : 0);
+                // spare / ne (both at most 32: the half keeps the product off the integers)
+                const int each = (int)(((float)spare + 0.5f) * __builtin_amdgcn_rcpf((float)ne));
+                q = each + (ie < spare - each * ne ? 1 : 0);
                 q = min(q, u.T - u.t - 1);
             }
-            // exclusive prefix sum of q over the joint list (lanes in list order)
-            int incl = q;
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1) {
-                const int v = __shfl_up(incl, d, kWave);
-                if (lane >= d) incl += v;
-            }
+            // prefix sum of q over the joint list (lanes in list order)
+            const int incl = wave_scan(q);
             if (fj) {
                 u.sbase = nj + incl - q;
                 u.sn = q;
@@ -844,11 +856,11 @@ __device__ __forceinline__ void build_lists(const KParams &p, Ctl &s, Utt &u) {
                     s.crow[u.sbase + o - 1] = c;
                 }
             }
-            total = __shfl(incl, kWave - 1, kWave);
+            total = __builtin_amdgcn_readlane(incl, kWave - 1);
         }
         if (lane == 0) {
             const int nl = __popcll(bl);
-            s.cnt = make_int4(nl, nj, nj + total, nl <= 1 ? 0 : 32 - __builtin_clz((unsigned)(nl - 1)));
+            s.cnt = make_int4(s.ok ? nl : -1, nj, nj + total, nl <= 1 ? 0 : 32 - __builtin_clz((unsigned)(nl - 1)));
         }
     }
     lds_sync();
@@ -1786,12 +1798,18 @@ __device__ __forceinline__ void lstm_and_pred(const KParams &p, Ctl &s, const Bu
 // every rank's keys knows that all of them are done with the iteration's staged
 // data.  A rank cannot overwrite a key before every workgroup has read it: it
 // stores the same half again two iterations on, after the keys of the next.
+// Where one wave's loads cover every rank (domains of few workgroups, few columns) wave 0, which
+// decides, gathers alone: no combining through LDS and no barrier before the decisions (with the
+// prefix sum of the spare columns by DPP: B=1 -2 % of a call, B=256 and B=512 -2 %).
 constexpr int kKeyRounds = 4;
 __device__ __forceinline__ void gather_keys(const KParams &p, Ctl &s, const Bufs &B, unsigned stamp, int ncol) {
     lds_sync();   // this workgroup's key stores have read s.wgkey
     const int P = s.P, nc = ncol, lane = threadIdx.x & (kWave - 1);
     const int lgp = nc <= 2 ? 0 : 31 - __builtin_clz((unsigned)(nc - 1));   // log2 of the column pairs, rounded up
-    const int pairs = 1 << lgp, cp = threadIdx.x & (pairs - 1), r0 = threadIdx.x >> lgp, step = kBlock >> lgp;
+    const int pairs = 1 << lgp, cp = threadIdx.x & (pairs - 1), r0 = threadIdx.x >> lgp;
+    const bool alone = P << lgp <= kWave * kKeyRounds;
+    if (alone && threadIdx.x >= kWave) return;
+    const int step = (alone ? kWave : kBlock) >> lgp;
     const unsigned dom = (stamp & 1) * p.n_dom + s.dom;
     const unsigned base = (dom * P * p.cols + 2 * cp) * 8u, stride = (unsigned)p.cols * 8u;
     const bool two = 2 * cp + 1 < nc, one = 2 * cp < nc;
@@ -1837,7 +1855,8 @@ __device__ __forceinline__ void gather_keys(const KParams &p, Ctl &s, const Bufs
         if (best0 != 0ull) atomicMax(&s.wgkey[2 * cp][0], best0);
         if (best1 != 0ull) atomicMax(&s.wgkey[2 * cp + 1][0], best1);
     }
-    lds_sync();
+    if (!alone) lds_sync();
+    else __atomic_signal_fence(__ATOMIC_SEQ_CST);   // (a wave's LDS operations complete in order)
 }
 
 // One utterance per lane of wave 0.  Its first decision is column u.col (frame t);
@@ -1966,7 +1985,7 @@ __device__ __forceinline__ void tap_copy(const KParams &p, Ctl &s) {
 }
 
 __device__ __forceinline__ void decide(const KParams &p, Ctl &s, Utt &u, unsigned stamp) {
-    if (threadIdx.x < kWave) decide_steps(p, s, u, stamp);
+    if (threadIdx.x < kWave && s.ok) decide_steps(p, s, u, stamp);
     if (p.logits) {
         lds_sync();
         tap_copy(p, s);
@@ -2181,6 +2200,10 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
     while (ok) {
         const int nl = __builtin_amdgcn_readfirstlane(s.cnt.x), nj = __builtin_amdgcn_readfirstlane(s.cnt.y),
                   ncol = __builtin_amdgcn_readfirstlane(s.cnt.z), lgn = __builtin_amdgcn_readfirstlane(s.cnt.w);
+        if (nl < 0) {
+            ok = false;
+            break;
+        }
         if (nl == 0 && nj == 0) break;
         if ((int)iter >= p.max_iter) {
             if (threadIdx.x == 0)
@@ -2215,10 +2238,6 @@ __global__ void __launch_bounds__(kBlock) decode_loop_kernel(KParams p) {
             gather_keys(p, s, B, iter, ncol);
             TLA(29);
             pmark(p, s, tlast, kPrKeys);
-            if (!s.ok) {   // (behind the gather's barrier: the same in every wave)
-                ok = false;
-                break;
-            }
             decide(p, s, u, iter);
         }
         if (nj == 0) lds_sync();   // (behind the keys' barrier otherwise)
