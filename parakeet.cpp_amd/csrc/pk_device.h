@@ -191,9 +191,9 @@ __device__ __forceinline__ void st_coh(float *p, float v) {
 
 // Workgroup barrier for LDS traffic only: each wave waits for its own LDS
 // operations (lgkmcnt 0) but not for its global loads and stores, which stay
-// in flight across it (s_barrier carries no implicit wait on gfx950).  Every
-// exchange between workgroups goes through dom_sync, which drains them.  The
-// signal fences keep the compiler from moving memory accesses across it.
+// in flight across it (s_barrier carries no implicit wait on gfx950); data of
+// other workgroups is waited for word by word.  The signal fences keep the
+// compiler from moving memory accesses across it.
 __device__ __forceinline__ void lds_sync() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0xC07F);   // gfx9 encoding: lgkmcnt(0), vmcnt and expcnt unconstrained
