@@ -357,7 +357,21 @@ int tile_matrix(const pk_tensor &t, int rows, int cols, const std::vector<int> *
 // symbol itself, only the address hipGetSymbolAddress returns for the current
 // device (kept per device in g_scratch).
 constexpr size_t kScratchBytes = (size_t)32 << 20;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// Room for the exchange buffers beyond what the 32 MiB limit counts for them (scratch_counted).
+constexpr size_t kScratchReserve = (size_t)16 << 20;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kScratchReserve];
+
+// What the limit of pk_decode_noalloc counts for flags, keys and exchange buffers: per workgroup
+// 256 B, per domain and column pair of shards of 8 ranks, per utterance two h, two c and two R rows
+// of each layer and one pp row.  Which batches fit is part of the interface; the buffers themselves
+// hold copies and row padding that depend on the plan.
+size_t scratch_counted(int nwg, int n_dom, int P, int m, int L, int H, int J) {
+    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    size_t shards = 1;
+    while (shards < 32 && shards * 8 < (size_t)P) shards *= 2;
+    return up(256 + (size_t)nwg * 256 + (size_t)2 * n_dom * kDomCap * shards * 16 + (n_dom == 1 ? (size_t)P * 64 : 0)) +
+           up(((size_t)12 * L * m * H + (size_t)m * J) * 4);
+}
 
 struct ScratchTable {
     std::mutex mu;
@@ -1444,6 +1458,11 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
     const size_t xchg = (xs + xc + xr + xh + xp) * 4;
     // the loop addresses the exchange buffers with 32-bit buffer offsets
     if (xchg >= (1ull << 31)) return fail(PK_ERR_UNSUPPORTED, "exchange buffers of %d utterances exceed 2 GiB", m);
+    if (cs.fixed) {
+        const size_t counted = scratch_counted(nwg, pl.n_dom, pl.P, m, L, H, J),
+                     taken = ((clear_bytes + 255) & ~(size_t)255) + ((xchg + 255) & ~(size_t)255);
+        if (taken > counted) cs.cap += std::min(taken - counted, kScratchReserve);
+    }
     if ((rc = cs.get(dec->d_xchg, xchg, &d_xchg))) return rc;
     p.hs = static_cast<float *>(d_xchg);
     p.cx = p.hs + xs;

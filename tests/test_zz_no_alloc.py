@@ -84,3 +84,32 @@ def test_noalloc_refuses_oversized_and_host_batches(tmp_path):
     for a in (frames_d, *out.values()):
         a.free()
     dec.close()
+
+
+def test_no_alloc_padded_exchange(tmp_path):
+    """A batch just past 256 sessions (17 utterances in some domains, exchange rows padded to 32) whose
+    counted buffers fit 32 MiB decodes without allocation, equal to the allocating call's tokens."""
+    from parakeet_amd import hipmem, pk, synth
+    path = str(tmp_path / "e.gguf")
+    synth.make_decoder_gguf(path, kind="eou", H=640, L=1, J=640, D=64, vocab=35, eou_id=33, eob_id=34, max_symbols=5,
+                            quant="q8_0")
+    n, T, cap = 257, 36, 240
+    dev = pk.Decoder.from_gguf(path, n_slots=n)
+    frames = synth.encoder_frames(5, n * T, 64)
+    enc = hipmem.DeviceArray.from_numpy(frames)
+    got = []
+    for noalloc in (False, True):
+        out = {k: hipmem.DeviceArray(4 * n * (cap if k in ("tokens", "segments") else 1))
+               for k in ("tokens", "n_tokens", "steps", "segments", "n_segments")}
+        for s in range(n):
+            dev.reset_state(s)
+        dev.decode_device(enc.ptr, np.arange(n) * T, np.full(n, T), np.arange(n), 5,
+                          {k: v.ptr for k, v in out.items()}, cap, noalloc=noalloc)
+        nt = out["n_tokens"].to_numpy(np.int32, n)
+        tk = out["tokens"].to_numpy(np.int32, n * cap).reshape(n, cap)
+        got.append([tk[u, :nt[u]].tolist() for u in range(n)])
+        for v in out.values():
+            v.free()
+    assert got[0] == got[1]
+    enc.free()
+    dev.close()
