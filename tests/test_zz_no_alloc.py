@@ -104,7 +104,7 @@ def test_no_alloc_padded_exchange(tmp_path):
         for s in range(n):
             dev.reset_state(s)
         dev.decode_device(enc.ptr, np.arange(n) * T, np.full(n, T), np.arange(n), 5,
-                          {k: v.ptr for k, v in out.items()}, cap, noalloc=noalloc)
+                          dict({k: v.ptr for k, v in out.items()}, seg_cap=cap), cap, noalloc=noalloc)
         nt = out["n_tokens"].to_numpy(np.int32, n)
         tk = out["tokens"].to_numpy(np.int32, n * cap).reshape(n, cap)
         got.append([tk[u, :nt[u]].tolist() for u in range(n)])
