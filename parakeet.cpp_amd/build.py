@@ -9,10 +9,11 @@
                           only where parakeet.cpp's sources are present: it compiles against the
                           reference's own src/parakeet_ctc.h (headers only, no ggml)
 
-  tests/cpp/oracle_asan, oracle_tsan, gguf_fuzz_asan
+  tests/cpp/oracle_asan, oracle_tsan, gguf_fuzz_asan, host_outputs_asan
                           host-only sanitizer builds (g++/gcc, no device code): the oracle under
-                          AddressSanitizer + UBSan and ThreadSanitizer, and the GGUF reader and
-                          decoder loader under a mutation fuzzer with AddressSanitizer + UBSan
+                          AddressSanitizer + UBSan and ThreadSanitizer, the GGUF reader and
+                          decoder loader under a mutation fuzzer with AddressSanitizer + UBSan, and
+                          the copy of results into a caller's arrays (csrc/host_outputs.h) with both
 
 Called by __graft_entry__.build(); every call recompiles.
 """
@@ -103,8 +104,8 @@ SAN_FLAGS = ["-O1", "-g", "-fno-omit-frame-pointer", "-fno-sanitize-recover=all"
 
 
 def build_sanitizers():
-    """Host code only, compiled by gcc / g++ (never hipcc): the oracle and its driver, and the
-    GGUF reader + decoder loader with the fuzz driver."""
+    """Host code only, compiled by gcc / g++ (never hipcc): the oracle and its driver, the copy of
+    results with its driver, and the GGUF reader + decoder loader with the fuzz driver."""
     oracle = os.path.join(ROOT, "oracle")
     cpp = os.path.join(ROOT, "tests", "cpp")
     outs = []
@@ -114,6 +115,11 @@ def build_sanitizers():
         _run(["gcc", "-std=c11", *SAN_FLAGS, san, f"-I{oracle}", *o_src, "-lm", "-lpthread", "-o", out + ".tmp"])
         os.replace(out + ".tmp", out)
         outs.append(out)
+    out = os.path.join(cpp, "host_outputs_asan")
+    _run(["g++", "-std=c++17", *SAN_FLAGS, "-fsanitize=address,undefined", f"-I{INC}", f"-I{CSRC}",
+          os.path.join(cpp, "host_outputs_main.cpp"), "-o", out + ".tmp"])
+    os.replace(out + ".tmp", out)
+    outs.append(out)
     if os.path.exists(os.path.join(HERE, "libparakeet_hip.so")):
         out = os.path.join(cpp, "gguf_fuzz_asan")
         srcs = [os.path.join(cpp, "gguf_fuzz_main.cpp")] + [os.path.join(CSRC, f) for f in

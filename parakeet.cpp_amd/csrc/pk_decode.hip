@@ -57,6 +57,7 @@
 extern char **environ;
 
 #include "parakeet_hip.h"
+#include "host_outputs.h"
 #include "pk_device.h"
 
 namespace {
@@ -1553,46 +1554,54 @@ relaunch:
     if (dec->timed) HIP_TRY(hipEventRecord(dec->ev[2], dec->stream));
     int *status = dec->h_pin.as<int>();   // read after the stream synchronisation below
     HIP_TRY(hipMemcpyAsync(status, p.status, 4 * sizeof(int), hipMemcpyDeviceToHost, dec->stream));
-    if (host) {
-        // Eager outputs are in pinned memory.  Larger ones copy the counters and control words
-        // first, then only each row's filled prefix.
+    // Eager outputs are in pinned memory.  Larger ones copy the counters and control words first,
+    // then only each row's filled prefix.
+    int *cnt = o_ntok;
+    int32_t *s_ctrl = o_ctrl;
+    std::vector<int> cnt_v;
+    if (host && !eager) {
+        if (dec->pin_cnt + 12 * (size_t)m <= dec->h_pin.n) {   // (m <= n_slots: slots are distinct)
+            cnt = reinterpret_cast<int *>(dec->h_pin.as<uint8_t>() + dec->pin_cnt);
+        } else {
+            cnt_v.resize(3 * (size_t)m);
+            cnt = cnt_v.data();
+        }
+        HIP_TRY(hipMemcpyAsync(cnt, o_ntok, 12 * (size_t)m, hipMemcpyDeviceToHost, dec->stream));
         const size_t cb = o_ctrl ? (size_t)m * PK_CTRL_N * 4 : 0;
-        std::vector<int> cnt_v;
-        int *cnt = o_ntok, *e_tok = o_tok, *e_seg = o_seg, *e_tr = o_trace;
-        int32_t *s_ctrl = o_ctrl;
-        if (!eager) {
-            if (dec->pin_cnt + 12 * (size_t)m <= dec->h_pin.n) {   // (m <= n_slots: slots are distinct)
-                cnt = reinterpret_cast<int *>(dec->h_pin.as<uint8_t>() + dec->pin_cnt);
-            } else {
-                cnt_v.resize(3 * (size_t)m);
-                cnt = cnt_v.data();
-            }
-            HIP_TRY(hipMemcpyAsync(cnt, o_ntok, 12 * (size_t)m, hipMemcpyDeviceToHost, dec->stream));
-            if ((rc = dec->h_out.ensure(std::max<size_t>(cb, 64)))) return rc;
+        if ((rc = dec->h_out.ensure(std::max<size_t>(cb, 64)))) return rc;
+        if (cb) {
             s_ctrl = dec->h_out.as<int32_t>();
-            if (cb) HIP_TRY(hipMemcpyAsync(s_ctrl, o_ctrl, cb, hipMemcpyDeviceToHost, dec->stream));
-            e_tok = e_seg = e_tr = nullptr;
+            HIP_TRY(hipMemcpyAsync(s_ctrl, o_ctrl, cb, hipMemcpyDeviceToHost, dec->stream));
         }
-        HIP_TRY(hipStreamSynchronize(dec->stream));
-        if (status[0] == pkdev::kStatusNotResident && !coop_retry) {   // nothing was decoded: again
-            if ((rc = after_not_resident(dec, p.status))) return rc;
-            coop_retry = true;
-            goto relaunch;
-        }
-        const int *c_tok = cnt, *c_steps = c_tok + m, *c_seg = c_steps + m;
-        // rows of width wt / ws / wr (prefix copies) or of the full capacities (eager)
-        int wt = tcap, ws = bt->segments ? scap : 0, wr = o_trace ? trcap : 0;
-        const int *s_tok = e_tok, *s_seg = e_seg, *s_tr = e_tr;
+    }
+    HIP_TRY(hipStreamSynchronize(dec->stream));
+    if (status[0] == pkdev::kStatusNotResident && !coop_retry) {   // nothing was decoded: again
+        if ((rc = after_not_resident(dec, p.status))) return rc;
+        coop_retry = true;
+        goto relaunch;
+    }
+    if (status[0] == pkdev::kStatusNotResident) return fail(PK_ERR_DEVICE, "decode loop grid not co-resident");
+    dec->last_iters = status[1];
+    // nothing a launch writes is read before its error word
+    pkhost::HostOutputs ho;
+    ho.bt = bt;
+    ho.map = map.data();
+    ho.m = m;
+    ho.tcap = tcap;
+    ho.scap = bt->segments ? scap : 0;
+    ho.trcap = o_trace ? trcap : 0;
+    ho.lsteps = o_logits ? lsteps : 0;
+    ho.Vo = p.Vo;
+    if ((rc = ho.accept(status, cnt))) return fail(rc, "device decode failed (status %d)", rc);
+    if (host) {
+        // rows of the full capacities (eager) or of the longest prefix
+        int wt = tcap, ws = ho.scap, wr = ho.trcap;
+        const int *s_tok = o_tok, *s_seg = o_seg, *s_tr = o_trace;
         std::vector<int> prefix;
         if (!eager) {
-            wt = ws = wr = 0;
-            for (int i = 0; i < m; ++i) {
-                wt = std::max(wt, std::min(c_tok[i], tcap));
-                ws = std::max(ws, std::min(c_seg[i], scap));
-                wr = std::max(wr, std::min(c_steps[i], trcap));
-            }
-            if (!bt->segments) ws = 0;
-            if (!o_trace) wr = 0;
+            wt = ho.widest(&pkhost::HostOutputs::tokens);
+            ws = ho.widest(&pkhost::HostOutputs::segments);
+            wr = ho.widest(&pkhost::HostOutputs::traced);
             const size_t stage = (size_t)m * (wt + ws + 2 * (size_t)wr) * 4;
             if (stage > 0) {
                 prefix.resize(stage / 4);
@@ -1612,42 +1621,14 @@ relaunch:
                 s_tr = p_tr;
             }
         }
-        if (o_ctrl)
-            for (int i = 0; i < m; ++i)
-                memcpy(bt->ctrl_out + (size_t)map[i] * PK_CTRL_N, s_ctrl + (size_t)i * PK_CTRL_N, PK_CTRL_N * 4);
+        ho.place(s_tok, wt, s_seg, ws, s_tr, wr, s_ctrl);
         if (o_logits)   // debug tap: the rows of the steps taken (utterance order may differ)
             for (int i = 0; i < m; ++i) {
-                const size_t taken = (size_t)std::min(c_steps[i], lsteps) * p.Vo * 4;
-                float *dst = bt->logits + (size_t)map[i] * lrow;
-                if (eager) memcpy(dst, o_logits + (size_t)i * lrow, taken);
-                else if (taken > 0) HIP_TRY(hipMemcpy(dst, o_logits + (size_t)i * lrow, taken, hipMemcpyDeviceToHost));
+                const size_t taken = ho.tap_bytes(i);
+                if (eager) memcpy(ho.tap_row(i), o_logits + (size_t)i * lrow, taken);
+                else if (taken > 0) HIP_TRY(hipMemcpy(ho.tap_row(i), o_logits + (size_t)i * lrow, taken, hipMemcpyDeviceToHost));
             }
-        for (int i = 0; i < m; ++i) {
-            const int u = map[i];
-            bt->n_tokens[u] = c_tok[i];
-            bt->steps[u] = c_steps[i];
-            const int nt = std::min(c_tok[i], tcap);
-            if (nt > 0) memcpy(bt->tokens + (size_t)u * tcap, s_tok + (size_t)i * wt, 4 * (size_t)nt);
-            if (bt->n_segments) bt->n_segments[u] = c_seg[i];
-            if (ws) {
-                const int ns = std::min(c_seg[i], scap);
-                if (ns > 0) memcpy(bt->segments + (size_t)u * scap, s_seg + (size_t)i * ws, 4 * (size_t)ns);
-            }
-            if (wr) {
-                const int ns = std::min(c_steps[i], trcap);
-                if (ns > 0) memcpy(bt->trace + (size_t)u * trcap * 2, s_tr + (size_t)i * wr * 2, 8 * (size_t)ns);
-            }
-        }
-    } else {
-        HIP_TRY(hipStreamSynchronize(dec->stream));
-        if (status[0] == pkdev::kStatusNotResident && !coop_retry) {   // nothing was decoded: again
-            if ((rc = after_not_resident(dec, p.status))) return rc;
-            coop_retry = true;
-            goto relaunch;
-        }
     }
-    if (status[0] == pkdev::kStatusNotResident) return fail(PK_ERR_DEVICE, "decode loop grid not co-resident");
-    dec->last_iters = status[1];
     if (prof) {
         unsigned long long t[pkdev::kPrN];
         HIP_TRY(hipMemcpy(t, dec->d_prof.p, sizeof t, hipMemcpyDeviceToHost));
@@ -1670,7 +1651,6 @@ relaunch:
             fprintf(stderr, "\n");
         }
     }
-    if (status[0]) return fail(status[0], "device decode failed (status %d)", status[0]);
     if (status[2]) return fail(PK_ERR_OVERFLOW, "token or segment capacity exceeded");
     return 0;
 }

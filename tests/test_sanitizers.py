@@ -12,6 +12,10 @@
   byte flips, extreme values in header fields, inserted / removed bytes, on
   TDT and EOU seeds with q8_0 / q4_0 / f16 matrices.  A corrupt file must be
   rejected or accepted with every tensor inside the buffer, never crash.
+- The copy of a call's results into the caller's arrays (csrc/host_outputs.h) built
+  with AddressSanitizer + UBSan (tests/cpp/host_outputs_main.cpp): a launch that
+  ended with an error has written no counters, so whatever their place holds must
+  not become a length.
 
 The binaries are built by __graft_entry__.build() with gcc / g++ only."""
 import json
@@ -53,3 +57,7 @@ def test_gguf_reader_fuzz(tmp_path, model, quant):
         # both outcomes occur: the mutations reach past the header checks
         assert out["accepted"] > 500 and out["rejected"] > 500, out
         assert out["loaded"] > 0 and out["load_rejected"] > 0, out
+
+
+def test_host_outputs_of_failed_and_finished_launches():
+    assert _run([os.path.join(CPP, "host_outputs_asan")]).strip() == "ok"
