@@ -55,9 +55,15 @@ struct HostOutputs {
             if (ctrl) memcpy(bt->ctrl_out + u * PK_CTRL_N, ctrl + (size_t)i * PK_CTRL_N, PK_CTRL_N * 4);
         }
     }
-    // Bytes of utterance i's tapped steps (those it took), and their place in the caller's array.
-    size_t tap_bytes(int i) const { return (size_t)tapped(i) * Vo * 4; }
-    float *tap_row(int i) const { return bt->logits + (size_t)map[i] * lsteps * Vo; }
+    // Tapped steps k0 .. k0 + nk - 1 of utterances i0 .. i1 - 1, rows of nk steps at `rows`: those taken.
+    void place_tap(const float *rows, int i0, int i1, int k0, int nk) const {
+        for (int i = i0; i < i1; ++i) {
+            const int n = clamp(tapped(i) - k0, nk);
+            if (n > 0)
+                memcpy(bt->logits + ((size_t)map[i] * lsteps + k0) * Vo, rows + (size_t)(i - i0) * nk * Vo,
+                       (size_t)n * Vo * 4);
+        }
+    }
 };
 
 }  // namespace pkhost

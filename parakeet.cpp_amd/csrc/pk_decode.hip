@@ -81,6 +81,10 @@ constexpr int kMaxBatch = PK_MAX_BATCH;
 // results in host memory: 95 -> 88 us per call, with the frames and the descriptor block going up in
 // one copy; seven TDT-0.6b utterances with tapped logits -3 %)
 constexpr size_t kEagerCopyBytes = 256 << 10;
+// larger tapped logits come back through a pinned block of up to this size, many utterances to a
+// copy (one blocking copy per utterance costs 13 to 20 us: 300 EOU-120m sessions with one tapped step
+// took 6.3 ms a call)
+constexpr size_t kTapStage = 4 << 20;
 // host frames up to this size go up through a pinned staging block of the decoder
 constexpr size_t kPinnedFrames = 64ull << 20;
 // host frames up to this size go up in one copy with the descriptor block
@@ -429,6 +433,7 @@ struct pk_decoder {
     size_t pin_cnt = 0;        // offset of the counters in h_pin (the descriptor block ends there)
     HostBuf h_out;             // staging of host-memory outputs
     HostBuf h_frames;          // staging of host-memory frames (up to kPinnedFrames bytes)
+    HostBuf h_tap;             // staging of tapped logits (up to kTapStage bytes, or one step's)
     unsigned char *scratch = nullptr;   // this device's fixed scratch array (pk_decode_noalloc)
     int last_iters = 0;
     // a call decoded in several launches (decode_chained): the kernels' times and the
@@ -445,7 +450,7 @@ struct pk_decoder {
             b->p = nullptr;
             b->n = 0;
         }
-        for (HostBuf *b : {&h_pin, &h_out, &h_frames}) {
+        for (HostBuf *b : {&h_pin, &h_out, &h_frames, &h_tap}) {
             b->p = nullptr;
             b->n = 0;
         }
@@ -1395,12 +1400,18 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
     int *o_tok, *o_ntok, *o_steps, *o_seg = nullptr, *o_nseg = nullptr, *o_trace = nullptr, *o_ctrl = nullptr;
     float *o_logits = nullptr;
     // host outputs of up to kEagerCopyBytes: the kernel writes them (each word once) straight into
-    // pinned memory and the call copies nothing back; larger ones go through device staging
-    const size_t out_words = (size_t)m * tcap + 3 * (size_t)m + (size_t)m * scap + (size_t)m * trcap * 2 +
-                             (size_t)m * PK_CTRL_N + (size_t)m * lrow;
-    const bool eager = host && (out_words - (3 + PK_CTRL_N) * (size_t)m) * 4 <= kEagerCopyBytes;
+    // pinned memory and the call copies nothing back; larger ones go through device staging.  The
+    // tapped logits join the others there while both fit and take the device staging by themselves
+    // otherwise.
+    const size_t row_words = (size_t)m * tcap + (size_t)m * scap + (size_t)m * trcap * 2,
+                 word_counts = (3 + PK_CTRL_N) * (size_t)m, tap_words = (size_t)m * lrow;
+    const bool eager = host && row_words * 4 <= kEagerCopyBytes,
+               tap_eager = eager && (row_words + tap_words) * 4 <= kEagerCopyBytes;
     if (host) {
-        if ((rc = eager ? dec->h_out.ensure(std::max(out_words * 4, kEagerCopyBytes)) : dec->d_out.ensure(out_words * 4 + 64))) return rc;
+        const size_t pinned = (eager ? row_words + word_counts : 0) + (tap_eager ? tap_words : 0),
+                     staged = (eager ? 0 : row_words + word_counts) + (tap_eager ? 0 : tap_words);
+        if (eager && (rc = dec->h_out.ensure(std::max(pinned * 4, kEagerCopyBytes)))) return rc;
+        if (staged > 0 && (rc = dec->d_out.ensure(staged * 4 + 64))) return rc;
         int *o = eager ? dec->h_out.as<int>() : dec->d_out.as<int>();
         o_tok = o; o += (size_t)m * tcap;
         o_ntok = o; o += m;
@@ -1409,6 +1420,7 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
         o_seg = scap > 0 ? o : nullptr; o += (size_t)m * scap;
         o_trace = trcap > 0 ? o : nullptr; o += (size_t)m * trcap * 2;
         o_ctrl = bt->ctrl_out ? o : nullptr; o += (size_t)m * PK_CTRL_N;
+        if (eager && !tap_eager) o = dec->d_out.as<int>();
         o_logits = lrow > 0 ? reinterpret_cast<float *>(o) : nullptr;
     } else {
         o_tok = bt->tokens; o_ntok = bt->n_tokens; o_steps = bt->steps;
@@ -1622,12 +1634,23 @@ relaunch:
             }
         }
         ho.place(s_tok, wt, s_seg, ws, s_tr, wr, s_ctrl);
-        if (o_logits)   // debug tap: the rows of the steps taken (utterance order may differ)
-            for (int i = 0; i < m; ++i) {
-                const size_t taken = ho.tap_bytes(i);
-                if (eager) memcpy(ho.tap_row(i), o_logits + (size_t)i * lrow, taken);
-                else if (taken > 0) HIP_TRY(hipMemcpy(ho.tap_row(i), o_logits + (size_t)i * lrow, taken, hipMemcpyDeviceToHost));
-            }
+        if (tap_eager) {   // debug tap: the rows of the steps taken (utterance order may differ)
+            ho.place_tap(o_logits, 0, m, 0, lsteps);
+        } else if (const int wide = o_logits ? ho.widest(&pkhost::HostOutputs::tapped) : 0) {
+            // through pinned memory, as many utterances and steps at a time as it takes
+            const size_t step = (size_t)p.Vo * 4;
+            const int ks = std::min<int>(wide, std::max<size_t>(kTapStage / step, 1)),
+                      us = std::min<int>(m, std::max<size_t>(kTapStage / (step * ks), 1));
+            if ((rc = dec->h_tap.ensure(step * ks * us))) return rc;
+            for (int k0 = 0; k0 < wide; k0 += ks)
+                for (int i0 = 0; i0 < m; i0 += us) {
+                    const int nk = std::min(ks, wide - k0), i1 = std::min(m, i0 + us);
+                    HIP_TRY(hipMemcpy2DAsync(dec->h_tap.p, step * nk, o_logits + (size_t)i0 * lrow + (size_t)k0 * p.Vo,
+                                             lrow * 4, step * nk, i1 - i0, hipMemcpyDeviceToHost, dec->stream));
+                    HIP_TRY(hipStreamSynchronize(dec->stream));
+                    ho.place_tap(dec->h_tap.as<float>(), i0, i1, k0, nk);
+                }
+        }
     }
     if (prof) {
         unsigned long long t[pkdev::kPrN];

@@ -77,9 +77,19 @@ struct Staged {
     }
 };
 
-void copy_back(const pkhost::HostOutputs &o, const Staged &s, int wt, int ws, int wr) {
+// ks, us: tapped steps and utterances staged at a time (0: all in place)
+void copy_back(const pkhost::HostOutputs &o, const Staged &s, int wt, int ws, int wr, int ks, int us) {
     o.place(s.tok.data(), wt, s.seg.data(), ws, s.tr.data(), wr, s.ctrl.data());
-    for (int i = 0; i < kM; ++i) memcpy(o.tap_row(i), s.logits.data() + (size_t)i * kSteps * kVo, o.tap_bytes(i));
+    if (ks == 0) return o.place_tap(s.logits.data(), 0, kM, 0, kSteps);
+    const int wide = o.widest(&pkhost::HostOutputs::tapped);
+    for (int k0 = 0; k0 < wide; k0 += ks)
+        for (int i0 = 0; i0 < kM; i0 += us) {
+            const int nk = std::min(ks, wide - k0), i1 = std::min(kM, i0 + us);
+            std::vector<float> rows;
+            for (int i = i0; i < i1; ++i)
+                for (int k = 0; k < nk * kVo; ++k) rows.push_back(s.logits[((size_t)i * kSteps + k0) * kVo + k]);
+            o.place_tap(rows.data(), i0, i1, k0, nk);
+        }
 }
 
 // Counters that a failed launch left as an earlier call's words: a trace's -1, logit bits, capacities.
@@ -94,17 +104,20 @@ int failed_launch() {
             CHECK(o.accept(status, counters.data()) == code);
             CHECK(o.widest(&pkhost::HostOutputs::tokens) == 0 && o.widest(&pkhost::HostOutputs::segments) == 0);
             CHECK(o.widest(&pkhost::HostOutputs::traced) == 0 && o.widest(&pkhost::HostOutputs::tapped) == 0);
-            copy_back(o, Staged(kTok, kSeg, kTr), kTok, kSeg, kTr);
+            copy_back(o, Staged(kTok, kSeg, kTr), kTok, kSeg, kTr, 0, 0);
             CHECK(c.untouched());
         }
     return 0;
 }
 
-// A finished launch: counters within and past the capacities, rows at full capacity and as prefixes.
+// A finished launch: counters within and past the capacities, rows at full capacity and as prefixes,
+// the tap in place and staged in parts.
 int finished_launch() {
     const std::vector<int> counters{3, 9, 0, /* steps */ 2, 6, 0, /* segments */ 1, 4, 0};
     const int status[4] = {0, 11, PK_ERR_OVERFLOW, 0};
-    for (bool prefix : {false, true}) {
+    const int stages[][2] = {{0, 0}, {1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 3}};
+    for (const auto &stage : stages) {
+        const bool prefix = stage[0] != 0;
         Caller c;
         pkhost::HostOutputs o = c.outputs();
         CHECK(o.accept(status, counters.data()) == 0);
@@ -112,7 +125,7 @@ int finished_launch() {
                   ws = prefix ? o.widest(&pkhost::HostOutputs::segments) : kSeg,
                   wr = prefix ? o.widest(&pkhost::HostOutputs::traced) : kTr;
         CHECK(wt == kTok && ws == kSeg && wr == kTr);
-        copy_back(o, Staged(wt, ws, wr), wt, ws, wr);
+        copy_back(o, Staged(wt, ws, wr), wt, ws, wr, stage[0], stage[1]);
         for (int u = 0; u < kN; ++u) {
             const int i = u == 2 ? 0 : u == 0 ? 1 : u == 3 ? 2 : -1;   // the launch's index of utterance u
             const int nt = i < 0 ? 0 : counters[i], ns = i < 0 ? 0 : counters[kM + i], ng = i < 0 ? 0 : counters[2 * kM + i];

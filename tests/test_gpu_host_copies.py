@@ -1,8 +1,9 @@
 """Host-memory calls around the sizes where their copies change: frames up with the descriptor block in
-one copy up to 1 MiB, outputs written straight into pinned memory up to 256 KiB (tokens, segments, trace
-and tapped logits together).  On either side of each line the results equal those of the same windows
-decoded from device frames with another split of the outputs, bit for bit, and the logit rows of steps an
-utterance does not reach stay untouched."""
+one copy up to 1 MiB, outputs written straight into pinned memory up to 256 KiB (tokens, segments and
+trace; the tapped logits too while all of them fit, and through pinned blocks of 4 MiB beyond).  On either
+side of each line the results equal those of the same windows decoded from device frames with another
+split of the outputs, bit for bit, and the logit rows of steps an utterance does not reach stay
+untouched."""
 import numpy as np
 import pytest
 
@@ -66,4 +67,32 @@ def test_outputs_line(tmp_path, extra):
         assert 0 < x["steps"] < steps
         assert not np.isnan(x["logits"][:x["steps"]]).any()
         assert np.isnan(x["logits"][x["steps"]:]).all()
+    dev.close()
+
+
+# n sessions, tapped steps, frames of the first and of the others: the tap just past the pinned line with the
+# tokens within it; several blocks of utterances (128 steps of 8,198 floats fit one); one utterance's steps in
+# two blocks beside one of a few steps; tokens past the pinned line as well
+@pytest.mark.parametrize("n,steps,first,rest,cap", [(8, 1, 3, 2, None), (150, 2, 2, 1, None), (2, 200, 120, 2, None),
+                                                    (40, 3, 2, 3, 2000)])
+def test_staged_tap(tmp_path, n, steps, first, rest, cap):
+    from parakeet_amd import pk, synth
+    path = str(tmp_path / "d.gguf")
+    synth.make_shape(path, "tdt-0.6b-v3")
+    dev = pk.Decoder.from_gguf(path, n_slots=n + 1)
+    encs = [synth.encoder_frames(80 + u, first if u == 0 else rest, dev.info.D) for u in range(n)]
+    print(f"{n} sessions, {steps} tapped steps", flush=True)
+    got = dev.decode(encs, logit_steps=steps, token_cap=cap)
+    assert max(x["steps"] for x in got) > 1
+    for u in sorted({0, 1, n // 2, 126 % n, 127 % n, n - 1}):
+        one = dev.decode([encs[u]], slots=[n], reset=[1], logit_steps=5)[0]   # into pinned memory by the kernel
+        assert one["steps"] == got[u]["steps"] and np.array_equal(one["tokens"], got[u]["tokens"])
+        k = min(steps, 5, one["steps"])
+        a, b = got[u]["logits"][:k], one["logits"][:k]
+        assert np.linalg.norm(a - b) <= 4e-6 * np.linalg.norm(b), u   # 32-bit sums in another order
+        taken = min(steps, got[u]["steps"])
+        assert not np.isnan(got[u]["logits"][:taken]).any() and np.isnan(got[u]["logits"][taken:]).all()
+        # each tapped step's argmax is its decision: steps past the fifth are in their place too
+        am = got[u]["logits"][:taken, :dev.info.V1].argmax(1)
+        assert [t for t in am.tolist() if t != dev.info.blank] == got[u]["tokens"][:np.sum(am != dev.info.blank)].tolist()
     dev.close()
