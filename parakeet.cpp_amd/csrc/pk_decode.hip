@@ -95,8 +95,8 @@ constexpr int kCacheMinFrames = 16;
 // measured faster up to 256 rows, slower from 750 on)
 constexpr long long kNarrowRows = 256;
 // enc_proj over at least this many rows runs the wide kernel (128 x 320 tiles; measured against the
-// 64 x 64 tiles with q8_0, f16 and f32 weights: 8,192 rows 51 / 55 us, 46 / 51, 61 / 66; 16,384 rows
-// 94 / 59, 87 / 56, 112 / 73)
+// 64 x 64 tiles with q8_0, f16 and f32 weights: 8,192 rows 47 / 47 us, 43 / 43, 57 / 58; 16,384 rows
+// 89 / 51, 83 / 48, 106 / 64)
 constexpr long long kWideRows = 10240;
 
 thread_local std::string g_err;

@@ -453,10 +453,14 @@ __device__ __forceinline__ f32x4 ep_mma(half8 a_h, half8 a_l, half8 b, half8 b_l
     }
     return acc;
 }
+// Bias of output column col (past the last: the last one's, never stored).  Loaded before the
+// products: behind the epilogue's stores, which may alias it, each load waits by itself (20 in a
+// wave of the wide kernel: 10,240 rows of TDT-0.6b q8_0 55 us instead of 47; 64 x 64 tiles, 4 in a
+// wave: 4,096 rows 36 instead of 34).
+__device__ __forceinline__ float ep_bias(const EncProj &e, int col) { return e.bias[min(col, e.J - 1)]; }
 // D fragment of a tile: a lane holds output column `col` of rows row .. row + 3.
-__device__ __forceinline__ void ep_store(const EncProj &e, long long row, int col, f32x4 acc) {
+__device__ __forceinline__ void ep_store(const EncProj &e, long long row, int col, f32x4 acc, float bc) {
     if (col >= e.J) return;
-    const float bc = e.bias[col];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
         if (row + i < e.rows) e.out[(size_t)(row + i) * e.J + col] = acc[i] + bc;
@@ -494,8 +498,12 @@ __global__ void __launch_bounds__(256) enc_proj_kernel(EncProj e) {
             if (tid < kEpTile) ws = e.w_scale[(size_t)(k0 / kEpK) * e.J + scol];
     };
     f32x4 acc[4];
+    float bias[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 4; ++t) {
+        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        bias[t] = ep_bias(e, n0 + t * 16 + (lane & 15));
+    }
     fetch(0);
     for (int k0 = 0; k0 < e.d_enc; k0 += kEpK) {
         {
@@ -525,24 +533,24 @@ __global__ void __launch_bounds__(256) enc_proj_kernel(EncProj e) {
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t)
-        ep_store(e, m0 + wave * 16 + (lane >> 4) * 4, n0 + t * 16 + (lane & 15), acc[t]);
+        ep_store(e, m0 + wave * 16 + (lane >> 4) * 4, n0 + t * 16 + (lane & 15), acc[t], bias[t]);
 }
 
 // Large row counts (batched offline decoding): workgroup of 128 output rows x
 // 320 outputs, 8 waves of 64 x 80 (4 x 5 tiles).  A frame is split and staged
 // J / 320 times instead of J / 64 times and read from LDS by 4 waves instead of
 // one per 4 tiles; per K step a wave reads 13 KB of fragments from LDS for 40
-// MFMAs (64 x 64 tiles: 6 KB for 12).  Two LDS buffers, one barrier per K step:
+// MFMAs (f32: 18 KB for 60), with 64 x 64 tiles 6 KB for 8 (f32: 10 KB for 12).  Two LDS buffers, one barrier per K step:
 // step k+1 is written from registers and step k+2's loads are issued before the
 // products of step k (loads one more step ahead measured the same).  Workgroups
 // that share rows sit on one XCD (ids 8 apart), one after the other, so the second
 // reads the frames from its L2.
-// 131,072 rows, D = 1024, J = 640: q8_0 481 us, f16 446 us, f32 605 us (0.71, 0.77,
-// 0.85 PFLOP/s of MFMA; a large library product reaches 1.21 on the same card), 1279,
-// 1285 and 1408 us with enc_proj_kernel.  It is bound by the workgroup's serial K
-// steps, about 1.5 us each, so a launch takes 50 us however few its rows are: up to
-// 8,192 rows the 64 x 64 tiles are as fast or faster (51 against 55 us; 16,384 rows:
-// 94 against 59), hence the host's line (kWideRows) between the two.
+// 131,072 rows, D = 1024, J = 640: q8_0 433 us, f16 384 us, f32 535 us (0.79, 0.89,
+// 0.96 PFLOP/s of MFMA; a large library product reaches 1.21 on the same card), 1245,
+// 1234 and 1375 us with enc_proj_kernel.  It is bound by the workgroup's serial K
+// steps, about 1.3 us each, so a launch takes 43 us however few its rows are: up to
+// 8,192 rows the 64 x 64 tiles are as fast or faster (47 us either way; 5,120 rows: 40
+// against 46; 16,384: 89 against 51), hence the host's line (kWideRows) between the two.
 constexpr int kEwRows = 128, kEwCols = 320, kEwThreads = 512;
 template <int W>
 __global__ void __launch_bounds__(kEwThreads) enc_proj_wide_kernel(EncProj e) {
@@ -593,10 +601,13 @@ __global__ void __launch_bounds__(kEwThreads) enc_proj_wide_kernel(EncProj e) {
             if (tid < kEwCols) bs[b][tid] = ws;
     };
     f32x4 acc[4][5];
+    float bias[5];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int n = 0; n < 5; ++n) {
+        bias[n] = ep_bias(e, n0 + wn + n * 16 + (lane & 15));
 #pragma unroll
-        for (int n = 0; n < 5; ++n) acc[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < 4; ++t) acc[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     const int steps = e.d_enc / kEpK, last = e.d_enc - kEpK;
     fetch(0);
     stage(0);
@@ -630,7 +641,7 @@ __global__ void __launch_bounds__(kEwThreads) enc_proj_wide_kernel(EncProj e) {
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int n = 0; n < 5; ++n)
-            ep_store(e, m0 + wr + t * 16 + (lane >> 4) * 4, n0 + wn + n * 16 + (lane & 15), acc[t][n]);
+            ep_store(e, m0 + wr + t * 16 + (lane >> 4) * 4, n0 + wn + n * 16 + (lane & 15), acc[t][n], bias[n]);
 }
 
 // Few rows (streaming chunks, short windows).  There the tiled kernels above run
@@ -679,6 +690,7 @@ __global__ void __launch_bounds__(256) enc_proj_narrow_kernel(EncProj e) {
         }
     };
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float bias = ep_bias(e, col);
     auto mul = [&](int b, const Batch &x) {
 #pragma unroll
         for (int s = 0; s < kEnSteps; ++s) {
@@ -696,7 +708,7 @@ __global__ void __launch_bounds__(256) enc_proj_narrow_kernel(EncProj e) {
         load(b + 2, X);
         if (b + 1 < nb) mul(b + 1, Y);
     }
-    ep_store(e, m0 + (lane >> 4) * 4, col, acc);
+    ep_store(e, m0 + (lane >> 4) * 4, col, acc, bias);
 }
 
 // ---------------------------------------------------------------- decode loop
