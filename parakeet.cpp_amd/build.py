@@ -9,6 +9,7 @@
                           only where parakeet.cpp's sources are present: it compiles against the
                           reference's own src/parakeet_ctc.h (headers only, no ggml)
 
+  tests/cpp/enc_proj_rule prints the enc_proj kernel that sizes take (csrc/enc_proj_rule.h; host only)
   tests/cpp/oracle_asan, oracle_tsan, gguf_fuzz_asan, host_outputs_asan
                           host-only sanitizer builds (g++/gcc, no device code): the oracle under
                           AddressSanitizer + UBSan and ThreadSanitizer, the GGUF reader and
@@ -100,6 +101,14 @@ def build_dropin_test():
     return out
 
 
+def build_rule_test():
+    out = os.path.join(ROOT, "tests", "cpp", "enc_proj_rule")
+    _run(["g++", "-O2", "-std=c++17", "-Wall", f"-I{CSRC}", os.path.join(ROOT, "tests", "cpp", "enc_proj_rule_main.cpp"),
+          "-o", out + ".tmp"])
+    os.replace(out + ".tmp", out)
+    return out
+
+
 SAN_FLAGS = ["-O1", "-g", "-fno-omit-frame-pointer", "-fno-sanitize-recover=all"]
 
 
@@ -133,7 +142,7 @@ def build_sanitizers():
 
 def build_all():
     return [build_hip(), build_decoder(), build_calib(), build_api_test("decoder_api_main", hip=True),
-            build_api_test("loader_main"), build_dropin_test(), *build_sanitizers()]
+            build_api_test("loader_main"), build_dropin_test(), build_rule_test(), *build_sanitizers()]
 
 
 if __name__ == "__main__":

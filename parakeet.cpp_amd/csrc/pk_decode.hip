@@ -8,8 +8,9 @@
 //                       once per window (src/parakeet_tdt.cpp:433-483 computes
 //                       the same projection as a ggml graph; the CPU path
 //                       recomputes it per step at :167-168).  At most
-//                       kNarrowRows rows: enc_proj_narrow_kernel, at least
-//                       kWideRows: enc_proj_wide_kernel (bit-identical outputs).
+//                       256 rows: enc_proj_narrow_kernel, for many rows
+//                       enc_proj_wide_kernel (see enc_proj_rule.h;
+//                       bit-identical outputs).
 //   decode_loop_kernel  all lockstep iterations of all utterances in one
 //                       launch (an ordinary dispatch whose workgroups first
 //                       check that the whole grid is resident, relaunched
@@ -57,6 +58,7 @@
 extern char **environ;
 
 #include "parakeet_hip.h"
+#include "enc_proj_rule.h"
 #include "host_outputs.h"
 #include "pk_device.h"
 
@@ -91,14 +93,6 @@ constexpr size_t kPinnedFrames = 64ull << 20;
 constexpr size_t kJoinedFrames = 1 << 20;
 // windows shorter than this many frames do not fill the LDS weight cache
 constexpr int kCacheMinFrames = 16;
-// enc_proj over at most this many rows runs the narrow kernel (one wave per 16x16 block;
-// measured faster up to 256 rows, slower from 750 on)
-constexpr long long kNarrowRows = 256;
-// enc_proj over at least this many rows runs the wide kernel (128 x 320 tiles; measured against the
-// 64 x 64 tiles with q8_0, f16 and f32 weights: 8,192 rows 47 / 47 us, 43 / 43, 57 / 58; 16,384 rows
-// 89 / 51, 83 / 48, 106 / 64)
-constexpr long long kWideRows = 10240;
-
 thread_local std::string g_err;
 
 // Decode-loop launches of this process, per device: the loop's workgroups
@@ -1176,6 +1170,8 @@ int after_not_resident(pk_decoder *dec, int *d_status) {
     return 0;
 }
 
+static_assert(pkhost::kTileEdge == pkdev::kEpTile && pkhost::kWideTileRows == pkdev::kEwRows &&
+                  pkhost::kWideTileCols == pkdev::kEwCols, "enc_proj_rule.h states the kernels' tiles");
 template <int W>
 void launch_enc_proj(char which, const pkdev::EncProj &e, hipStream_t st) {
     if (which == 'n') {
@@ -1381,7 +1377,7 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
         // tiles over the packed rows of all utterances; the kernel also clears the loop's words.
         // The kernels give bit-identical rows (PK_ENC_PROJ=narrow / tile / wide forces one).
         const char *ep_env = std::getenv("PK_ENC_PROJ");
-        const char which = ep_env ? ep_env[0] : rows <= kNarrowRows ? 'n' : rows < kWideRows ? 't' : 'w';
+        const char which = ep_env ? ep_env[0] : pkhost::enc_proj_kernel_for(rows, J, dec->n_cu);
         pkdev::EncProj ep{dec->w_enc_hi, dec->w_enc_lo, dec->w_enc_scale, dec->b_enc, enc, J, D, m, d_src, d_dst, rows,
                           d_encp, static_cast<unsigned *>(d_clear), clear_words};
         launch_enc_proj(dec->enc_w, which, ep, dec->stream);

@@ -550,7 +550,8 @@ __global__ void __launch_bounds__(256) enc_proj_kernel(EncProj e) {
 // 1234 and 1375 us with enc_proj_kernel.  It is bound by the workgroup's serial K
 // steps, about 1.3 us each, so a launch takes 43 us however few its rows are: up to
 // 8,192 rows the 64 x 64 tiles are as fast or faster (47 us either way; 5,120 rows: 40
-// against 46; 16,384: 89 against 51), hence the host's line (kWideRows) between the two.
+// against 46; 16,384: 89 against 51), and a launch of few columns leaves most of its
+// waves empty, hence the host's rule between the two (enc_proj_rule.h).
 constexpr int kEwRows = 128, kEwCols = 320, kEwThreads = 512;
 template <int W>
 __global__ void __launch_bounds__(kEwThreads) enc_proj_wide_kernel(EncProj e) {
