@@ -37,9 +37,9 @@ def _both(dev, encs, n, **kw):
 
 @pytest.mark.parametrize("B", [1, 2, 4, 40])
 def test_tdt_blank_runs_replay_and_equal(tmp_path, B):
-    """B=1 and B=2 run the one-domain loop, whose argmax exchange switches between
-    the per-workgroup key slots (at most 2 joint columns) and the sharded atomics
-    (spare columns in use) from one iteration to the next."""
+    """B=1 and B=2 run on one domain of every workgroup, whose keys one wave gathers while at
+    most 2 joint columns are live and all eight waves once spare columns are in use; with the
+    runs off every iteration takes the first form."""
     from parakeet_amd import gguf, pk, synth
     import oracle
     path = str(tmp_path / "m.gguf")
@@ -101,33 +101,84 @@ def test_tdt_blank_runs_across_windows(tmp_path):
     dev.close()
 
 
-@pytest.mark.parametrize("B", [1, 2])
-def test_argmax_slots_equal_sharded_atomics(tmp_path, B):
-    """One-domain launches exchange the argmax keys through per-workgroup slots
-    while at most 2 joint columns are live; PK_ARGMAX_SLOTS=0 runs the same decode
-    with the sharded atomics and barrier.  Tokens, steps, traces and final state
-    are bit-identical, with and without runs of blanks (which switch the exchange
-    between the two forms from one iteration to the next)."""
-    from parakeet_amd import pk, synth
+def _lockstep(traces, T, durations, blank, max_symbols):
+    """Joint columns of each lockstep iteration of one domain, from its utterances' decisions (T in
+    the domain's order): one column per utterance with frames left, and the 16-column tile's spare
+    ones dealt out evenly as later frames of the utterances whose last decision was a blank."""
+    n = len(T)
+    t, sym, step = [0] * n, [0] * n, [0] * n
+    pend, keep = [True] * n, [False] * n
+    cols = []
+    while any(pend) or any(t[u] < T[u] for u in range(n)):
+        live = [u for u in range(n) if t[u] < T[u]]
+        spare = -len(live) % 16
+        runs = [u for u in live if keep[u]] if spare else []
+        ahead = [0] * n
+        for i, u in enumerate(runs):
+            q = spare // len(runs) + (1 if i < spare % len(runs) else 0)
+            ahead[u] = min(q, T[u] - t[u] - 1)
+        cols.append(len(live) + sum(ahead))
+        pend = [False] * n
+        for u in live:
+            t0 = t[u]
+            while True:
+                tok, d = traces[u][step[u]]
+                step[u] += 1
+                dur = durations[d]
+                keep[u] = tok == blank
+                if tok == blank:
+                    t[u], sym[u] = t[u] + max(1, dur), 0
+                else:
+                    pend[u], sym[u] = True, sym[u] + 1
+                    if dur > 0 or sym[u] >= max_symbols:
+                        t[u], sym[u] = t[u] + max(1, dur), 0
+                if not keep[u] or t[u] >= T[u] or t[u] - t0 > ahead[u]:
+                    break
+    assert step == [len(x) for x in traces]
+    return cols
+
+
+@pytest.mark.parametrize("B,domains", [(1, 1), (2, 1), (5, 1), (20, 2), (40, 4)])
+def test_key_gather_line(tmp_path, B, domains):
+    """The argmax keys of an iteration are gathered by one wave while its loads cover every
+    workgroup of the domain (P workgroups, column pairs rounded up to a power of two, P times pairs
+    at most 256) and by all eight waves beyond.  Each launch here has iterations on both sides of
+    that line, in an order that changes with the utterances' blanks; every decision replays
+    through the oracle, its tapped logits included, and the iterations are those the decisions
+    imply."""
+    from parakeet_amd import gguf, pk, synth
+    import oracle
+    from parity import rel
     path = str(tmp_path / "m.gguf")
     small_tdt(path)
-    dev = pk.Decoder.from_gguf(path, n_slots=8 * B)
-    encs = [synth.encoder_frames(1500 + u, 45 + 9 * u, 128) for u in range(B)]
-    for k, bias in enumerate((0.0, 3.0)):
-        bb = np.full(B, bias, np.float32)
-        base = 4 * B * k
-        os.environ["PK_ARGMAX_SLOTS"] = "0"
-        try:
-            ref = dev.decode(encs, slots=list(range(base + B, base + 2 * B)), trace=True, blank_bias=bb, max_symbols=5)
-        finally:
-            os.environ.pop("PK_ARGMAX_SLOTS", None)
-        got = dev.decode(encs, slots=list(range(base, base + B)), trace=True, blank_bias=bb, max_symbols=5)
-        for u in range(B):
-            assert np.array_equal(got[u]["tokens"], ref[u]["tokens"]), (bias, u)
-            assert np.array_equal(got[u]["trace"], ref[u]["trace"]), (bias, u)
-            assert got[u]["steps"] == ref[u]["steps"], (bias, u)
-            a, b = dev.read_state(base + u), dev.read_state(base + B + u)
-            assert np.array_equal(a["h"], b["h"]) and np.array_equal(a["c"], b["c"]), (bias, u)
+    dev = pk.Decoder.from_gguf(path, n_slots=B)
+    om = oracle.OracleModel.from_gguf(path, gguf)
+    P = pk.device_info()["n_cu"] // domains
+    T = [70 - (u // domains) * 60 // max(1, (B - 1) // domains) for u in range(B)]   # ends one after the other
+    encs = [synth.encoder_frames(1500 + u, T[u], 128) for u in range(B)]
+    bb = np.array([(1.5, 0.0, 3.0)[(u // domains) % 3] for u in range(B)], np.float32)
+    print(f"key gather: B={B} on {domains} domain(s) of {P}", flush=True)
+    TAP = 40
+    got = dev.decode(encs, trace=True, blank_bias=bb, max_symbols=5, logit_steps=TAP)
+    iters = 0
+    one_wave, all_waves = set(), set()
+    order = sorted(range(B), key=lambda u: -T[u])   # longest first, dealt round robin
+    for d in range(domains):
+        us = order[d::domains]
+        cols = _lockstep([got[u]["trace"].tolist() for u in us], [T[u] for u in us], [0, 1, 2, 3, 4], dev.info.blank, 5)
+        iters = max(iters, len(cols))
+        for c in cols:
+            pairs = 1 if c <= 2 else 1 << ((c - 1).bit_length() - 1)
+            if c:
+                (one_wave if P * pairs <= 256 else all_waves).add(c)
+    print(f"  columns gathered by one wave {sorted(one_wave)}, by all {sorted(all_waves)}", flush=True)
+    assert one_wave and all_waves and min(all_waves) > max(one_wave)
+    assert dev.last_timing()["iterations"] == iters
+    for u in range(B):
+        check_window(om, dev, u, encs[u], got[u], om.new_state(), 5, blank_bias=float(bb[u]))
+        n = min(TAP, got[u]["steps"])
+        rep = om.replay_window(encs[u], om.new_state(), 5, got[u]["trace"], blank_bias=float(bb[u]), n_tap=TAP)
+        assert all(rel(got[u]["logits"][j], rep["logits"][j]) < 1e-3 for j in range(n)), u
     dev.close()
 
 
