@@ -9,7 +9,8 @@
                           only where parakeet.cpp's sources are present: it compiles against the
                           reference's own src/parakeet_ctc.h (headers only, no ggml)
 
-  tests/cpp/enc_proj_rule prints the enc_proj kernel that sizes take (csrc/enc_proj_rule.h; host only)
+  tests/cpp/enc_proj_rule, exchange_word
+                          host-only drivers of csrc/enc_proj_rule.h and csrc/exchange_word.h
   tests/cpp/oracle_asan, oracle_tsan, gguf_fuzz_asan, host_outputs_asan
                           host-only sanitizer builds (g++/gcc, no device code): the oracle under
                           AddressSanitizer + UBSan and ThreadSanitizer, the GGUF reader and
@@ -101,9 +102,10 @@ def build_dropin_test():
     return out
 
 
-def build_rule_test():
-    out = os.path.join(ROOT, "tests", "cpp", "enc_proj_rule")
-    _run(["g++", "-O2", "-std=c++17", "-Wall", f"-I{CSRC}", os.path.join(ROOT, "tests", "cpp", "enc_proj_rule_main.cpp"),
+def build_header_test(name):
+    """tests/cpp/<name>: host-only driver of one of csrc's headers (g++)."""
+    out = os.path.join(ROOT, "tests", "cpp", name)
+    _run(["g++", "-O2", "-std=c++17", "-Wall", f"-I{CSRC}", os.path.join(ROOT, "tests", "cpp", name + "_main.cpp"),
           "-o", out + ".tmp"])
     os.replace(out + ".tmp", out)
     return out
@@ -142,7 +144,8 @@ def build_sanitizers():
 
 def build_all():
     return [build_hip(), build_decoder(), build_calib(), build_api_test("decoder_api_main", hip=True),
-            build_api_test("loader_main"), build_dropin_test(), build_rule_test(), *build_sanitizers()]
+            build_api_test("loader_main"), build_dropin_test(), build_header_test("enc_proj_rule"),
+            build_header_test("exchange_word"), *build_sanitizers()]
 
 
 if __name__ == "__main__":

@@ -9,6 +9,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include "exchange_word.h"
 #include "parakeet_hip.h"
 
 namespace pkdev {
@@ -28,7 +29,6 @@ constexpr int kFlagStride = 32;             // words between barrier flags (128 
 // error word of a launch whose ordinary dispatch was not co-resident (never returned to a caller:
 // the host relaunches the call cooperatively)
 constexpr int kStatusNotResident = 0x7001;
-constexpr unsigned kEmpty = 0xffffffffu;     // exchange word not written yet (a NaN no producer stores)
 constexpr int kKPad = 8;                    // halves of padding per staged row (bank spread)
 
 // Flags in the per-utterance control word.
@@ -944,14 +944,10 @@ __device__ __forceinline__ bool dom_sync(const KParams &p, Ctl &s, unsigned &epo
 // waits for all of its own stores before that, so a workgroup that has seen
 // every key sees every word emptied or written in the iteration.
 
-// A produced word: never the empty pattern (a NaN that loses one payload bit).
-__device__ __forceinline__ float filled(float v) {
-    const unsigned b = __float_as_uint(v);
-    return __uint_as_float(b == kEmpty ? b - 1u : b);
-}
+// (exchange_word.h: kEmpty, filled_word, any_empty)
+__device__ __forceinline__ float filled(float v) { return __uint_as_float(filled_word(__float_as_uint(v))); }
 __device__ __forceinline__ bool has_empty(float4 v) {
-    return max(max(__float_as_uint(v.x), __float_as_uint(v.y)),
-               max(__float_as_uint(v.z), __float_as_uint(v.w))) == kEmpty;
+    return any_empty(__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w));
 }
 __device__ __forceinline__ float4 empty4() {
     const float e = __uint_as_float(kEmpty);
