@@ -202,11 +202,13 @@ PK_API int pk_window_split(int32_t n_utts, const int32_t *n_frames, int32_t max_
  * serving loops, harnesses that forbid hipMalloc).  batch->mem must be
  * PK_MEM_DEVICE (frames and outputs already in device memory).  Every device
  * buffer of the call beyond its inputs and outputs (descriptors, enc_proj rows,
- * barrier flags, argmax keys, exchange buffers) comes from one fixed 32 MiB
- * array per device, held until the process ends; a batch that needs more is
- * refused with PK_ERR_UNSUPPORTED (about 16,000 frames x 640 joint units at
- * 64 utterances).  All calls on one device share that array: two calls that
- * overlap in time on the same device race. */
+ * barrier flags, argmax keys, exchange buffers) comes from one fixed array per
+ * device, held until the process ends: 32 MiB for what a batch may need, and
+ * 16 MiB in reserve for row padding of the exchange buffers, 48 MiB in all.  A
+ * batch that needs more than the 32 MiB is refused with PK_ERR_UNSUPPORTED (64
+ * utterances of a decoder with two layers of 640 units and 640 joint units:
+ * about 11,900 frames fit).  All calls on one device share that array: two calls
+ * that overlap in time on the same device race. */
 PK_API int pk_decode_noalloc(pk_decoder *dec, const pk_batch *batch);
 /* Time, with HIP events on the handle's stream, the last pk_decode's
  * kernels: enc_proj GEMM and the decode loop (milliseconds), and its lockstep

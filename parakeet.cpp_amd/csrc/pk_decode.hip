@@ -356,14 +356,16 @@ int tile_matrix(const pk_tensor &t, int rows, int cols, const std::vector<int> *
 // symbol itself, only the address hipGetSymbolAddress returns for the current
 // device (kept per device in g_scratch).
 constexpr size_t kScratchBytes = (size_t)32 << 20;
-// Room for the exchange buffers beyond what the 32 MiB limit counts for them (scratch_counted).
+// Room for the exchange buffers beyond what the 32 MiB limit counts for them (scratch_counted): 48 MiB
+// of device memory per device in all.
 constexpr size_t kScratchReserve = (size_t)16 << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes + kScratchReserve];
 
-// What the limit of pk_decode_noalloc counts for flags, keys and exchange buffers: per workgroup
-// 256 B, per domain and column pair of shards of 8 ranks, per utterance two h, two c and two R rows
-// of each layer and one pp row.  Which batches fit is part of the interface; the buffers themselves
-// hold copies and row padding that depend on the plan.
+// What the limit of pk_decode_noalloc counts at most for flags, keys and exchange buffers: per
+// workgroup 256 B, per domain and column pair of shards of 8 ranks, per utterance two h, two c and
+// two R rows of each layer and one pp row.  A batch that fits with these counted is taken whatever
+// the buffers' copies and row padding come to (up to the reserve), since which batches fit is part
+// of the interface; where the buffers are smaller (two layers and more), a few frames more fit.
 size_t scratch_counted(int nwg, int n_dom, int P, int m, int L, int H, int J) {
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     size_t shards = 1;
@@ -1468,6 +1470,8 @@ int decode_impl(pk_decoder *dec, const pk_batch *bt, bool keep_empty, CallScratc
     // the loop addresses the exchange buffers with 32-bit buffer offsets
     if (xchg >= (1ull << 31)) return fail(PK_ERR_UNSUPPORTED, "exchange buffers of %d utterances exceed 2 GiB", m);
     if (cs.fixed) {
+        // (what came before the exchange buffers has not grown by as much as their own count, so a
+        // batch that fits has not been refused above)
         const size_t counted = scratch_counted(nwg, pl.n_dom, pl.P, m, L, H, J),
                      taken = ((clear_bytes + 255) & ~(size_t)255) + ((xchg + 255) & ~(size_t)255);
         if (taken > counted) cs.cap += std::min(taken - counted, kScratchReserve);

@@ -929,8 +929,10 @@ __device__ __forceinline__ bool dom_sync(const KParams &p, Ctl &s, unsigned &epo
 // words it stages until none of them is empty.  One device-coherent store and
 // the load that sees it replace the store, its acknowledgement, a barrier (flag
 // store, polls of every member's flag) and the staging load behind it.  Layouts
-// give each producer whole lines: a tile's rows are stored by one wave, so no
-// line is invalidated under its readers by another workgroup's store.
+// give each producer whole lines of 128 bytes: a tile's rows are stored by one
+// wave, so no line is invalidated under its readers by another workgroup's store.
+// (The prediction output of a domain of one utterance is the exception: a tile is
+// then 64 bytes, and two neighbouring ranks share a line.)
 // Measured per exchange with nothing else in flight (store, wait, staged rows):
 // 16 rows over 64 workgroups 1.84 us against 2.71 us with a barrier, over 16
 // workgroups 2.07 against 2.57, one row over 256 workgroups 1.75 against 2.15.
@@ -1459,8 +1461,6 @@ __device__ __forceinline__ void cache_matrix(const TMat &m, int rank, int P, uns
     }
 }
 
-// Joint + argmax for this workgroup's output tiles.  Utterances are processed
-// 16 at a time (one MFMA column tile).
 // Row mapping of the joint's staging: a wave covers one pred tile (16 values)
 // of 16 columns, 1 KB in a row of ppx; thread t takes column (t / 4) % 16,
 // values 4 (t % 4) .. +3 of pred tiles t / 64, t / 64 + 8, ...
@@ -1479,6 +1479,8 @@ __device__ __forceinline__ void encp_prefetch(const KParams &p, const Ctl &s, co
     }
 }
 
+// Joint + argmax for this workgroup's output tiles.  Utterances are processed
+// 16 at a time (one MFMA column tile).
 template <int WC>
 __device__ __forceinline__ void joint_phase(const KParams &p, Ctl &s, const Bufs &B, const Lds &S, unsigned stamp, int ncol,
                             const float4 (&epre)[kStageMax], unsigned long long &tlast) {
@@ -1797,8 +1799,6 @@ __device__ __forceinline__ void lstm_and_pred(const KParams &p, Ctl &s, const Bu
     }
 }
 
-// Apply the argmax results of iteration `stamp` to every utterance of the joint
-// list: src/parakeet_tdt.cpp:936-967 (TDT) and src/parakeet_eou.cpp:275-332 (EOU).
 // The domain's best key per joint column and head.  Token keys: lane groups of
 // `pairs` threads load two columns of one rank each (16 bytes) until both carry
 // this iteration's stamp, every rank of the domain; then the wave's maximum per
@@ -1868,6 +1868,8 @@ __device__ __forceinline__ void gather_keys(const KParams &p, Ctl &s, const Bufs
     else __atomic_signal_fence(__ATOMIC_SEQ_CST);   // (a wave's LDS operations complete in order)
 }
 
+// Apply the argmax results of iteration `stamp` to every utterance of the joint
+// list: src/parakeet_tdt.cpp:936-967 (TDT) and src/parakeet_eou.cpp:275-332 (EOU).
 // One utterance per lane of wave 0.  Its first decision is column u.col (frame t);
 // while the decision keeps the prediction output (a TDT blank; an EOU blank, <EOB>
 // or special piece) and the next frame's column was evaluated, the walk goes
