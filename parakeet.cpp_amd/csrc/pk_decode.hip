@@ -1088,7 +1088,7 @@ int open_loop_lock(int device) {
 // cooperative queue.  An ordinary dispatch checks it in the kernel
 // (pkdev::coresident).  Loops of this process are kept apart by the ordering
 // above, loops of other processes by the per-device lock (DeviceLoopLock); if
-// one overlaps anyway, the barriers' 2 s limit ends the launch with
+// one overlaps anyway, the 2 s limit of the loop's waits ends the launch with
 // PK_ERR_TIMEOUT.
 //
 // Arrival limit of an ordinary dispatch's co-residency check (a workgroup's start to the whole
@@ -1105,7 +1105,7 @@ constexpr int kCoopAfterAbort = 256;
 // kStatusNotResident and the call is relaunched with coop = true (decode_impl); the device's
 // next kCoopAfterAbort launches are cooperative.  Where the runtime refuses a cooperative launch
 // (another process holds the device's cooperative queue), the loop runs as an ordinary
-// dispatch without the check, and its barriers' 2 s limit is the last guard.
+// dispatch without the check, and the 2 s limit of its waits is the last guard.
 // PK_LOOP_DISPATCH=0 makes every launch cooperative, =1 every launch an ordinary dispatch (a
 // relaunch then without the check), as under a profiler;
 // PK_ARRIVE_US sets the arrival limit for tests of the relaunch: the first launch of a call is
