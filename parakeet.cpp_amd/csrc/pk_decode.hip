@@ -93,6 +93,7 @@ constexpr size_t kPinnedFrames = 64ull << 20;
 constexpr size_t kJoinedFrames = 1 << 20;
 // windows shorter than this many frames do not fill the LDS weight cache
 constexpr int kCacheMinFrames = 16;
+
 thread_local std::string g_err;
 
 // Decode-loop launches of this process, per device: the loop's workgroups
